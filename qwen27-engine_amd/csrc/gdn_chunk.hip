@@ -265,10 +265,9 @@ __global__ void __launch_bounds__(512) gdn_chunk_kernel(const float* __restrict_
   __shared__ __align__(16) float sKb[kNB][kC][kKP];
   __shared__ __align__(16) float sQb[kNB][kC][kKP];
   __shared__ float sVb[kNB][kC][kNC];
-  __shared__ __align__(16) float sgb[kNB][kC];
-  __shared__ float sbb[kNB][kC];
+  __shared__ __align__(16) float sg[kC];
   __shared__ float sTb[kNB][kC][kPP], sMb[kNB][kC][kPP];  // Tinv and M, unpacked from P
-  __shared__ float sgam[2][kC], sdec[2][kC];              // decays of chunks n and n + 1
+  __shared__ float sgam[2][kC], sdec[2][kC], sbb[2][kC];  // decays and beta of chunks n and n + 1
   __shared__ __align__(16) v4f part[8][4][64];            // K S, Q S partial tiles (two token tiles each)
   __shared__ float sDl[2][kC][kDP];                       // Delta of the two column halves
   const int h = blockIdx.x, kh = h % HK, cg = blockIdx.y;
@@ -295,27 +294,42 @@ __global__ void __launch_bounds__(512) gdn_chunk_kernel(const float* __restrict_
   const int st_t = tid >> 5, st_e4 = (tid & 31) * 4, st_c = tid & 31;
   float4 pk[2], pq[2];
   float pv[2], pt[2], pg = 0.0f, pb = 0.0f;
-  auto fetch = [&](int ch) {  // chunk ch's rows into registers (zeros, and no loads, past T)
+  // Chunk ch's rows into registers, through buffer descriptors of the chunk's rows: reads past its last token return
+  // zeros, so no load is conditional and the compiler's waits count them exactly.
+  auto rows_of = [&](const float* p, int c0, int n, int ld, int width) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(p + (n > 0 ? (size_t)c0 * ld : 0)), 0, n > 0 ? ((n - 1) * ld + width) * 4 : 0,
+                                             0x00027000);
+  };
+  auto fetch = [&](int ch) {
     const int c0 = ch * kC, n = min(kC, T - c0);
+    const auto fk = rows_of(k + kh * 128, c0, n, stride, 128), fq = rows_of(q + kh * 128, c0, n, stride, 128);
+    const auto fv = rows_of(v + h * 128 + cg * kNC, c0, n, stride, kNC);
+    // P: parked in o's rows for a full chunk, else in the output plane (column st_c, key t)
+    const bool full = n == kC;
+    const auto fp = full ? rows_of(o + h * 128 + cg * kNC, c0, n, H * 128, kNC)
+                         : __builtin_amdgcn_make_buffer_rsrc(
+                               (void*)(planes + (size_t)pout * plane_sz + ((size_t)h * 128 + cg * kNC) * 128), 0,
+                               n > 0 ? kNC * 128 * 4 : 0, 0x00027000);
+    const int pl = full ? (st_t * H * 128 + st_c) * 4 : (st_c * 128 + st_t) * 4, ps = full ? 16 * H * 128 * 4 : 16 * 4;
 #pragma unroll
     for (int u = 0; u < 2; u++) {
-      const int t = st_t + 16 * u;
-      pk[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-      pq[u] = pk[u];
-      pv[u] = 0.0f;
-      pt[u] = 0.0f;
-      if (t < n) {
-        pk[u] = ld4(k + (size_t)(c0 + t) * stride + kh * 128 + st_e4);
-        pq[u] = ld4(q + (size_t)(c0 + t) * stride + kh * 128 + st_e4);
-        pv[u] = v[(size_t)(c0 + t) * stride + h * 128 + cg * kNC + st_c];
-      }
-      if (n == kC) pt[u] = o[((size_t)(c0 + t) * H + h) * 128 + cg * kNC + st_c];  // P, parked in o
-      else if (n > 0) pt[u] = planes[(size_t)pout * plane_sz + ((size_t)h * 128 + cg * kNC + st_c) * 128 + t];
+      const v4f a = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(fk, (st_t * stride + st_e4) * 4, 16 * u * stride * 4, 0));
+      const v4f b = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(fq, (st_t * stride + st_e4) * 4, 16 * u * stride * 4, 0));
+      pk[u] = make_float4(a[0], a[1], a[2], a[3]);
+      pq[u] = make_float4(b[0], b[1], b[2], b[3]);
+      const uint32_t c = __builtin_amdgcn_raw_buffer_load_b32(fv, (st_t * stride + st_c) * 4, 16 * u * stride * 4, 0);
+      const uint32_t d = __builtin_amdgcn_raw_buffer_load_b32(fp, pl, u * ps, 0);
+      pv[u] = __builtin_bit_cast(float, c);
+      pt[u] = __builtin_bit_cast(float, d);
     }
-    if (w == 1 && l < kC) {
-      pg = l < n ? g[(size_t)(c0 + l) * H + h] : 0.0f;
-      pb = l < n ? beta[(size_t)(c0 + l) * H + h] : 0.0f;
-    }
+  };
+  auto fetch_g = [&](int ch) {  // wave 1: g and beta, token l on lane l
+    const int c0 = ch * kC, n = min(kC, T - c0);
+    const auto fg = rows_of(g + h, c0, n, H, 1), fb = rows_of(beta + h, c0, n, H, 1);
+    const uint32_t a = __builtin_amdgcn_raw_buffer_load_b32(fg, l * H * 4, 0, 0);
+    const uint32_t b = __builtin_amdgcn_raw_buffer_load_b32(fb, l * H * 4, 0, 0);
+    pg = __builtin_bit_cast(float, a);
+    pb = __builtin_bit_cast(float, b);
   };
   auto stash = [&](int buf) {
 #pragma unroll
@@ -327,14 +341,14 @@ __global__ void __launch_bounds__(512) gdn_chunk_kernel(const float* __restrict_
       sMb[buf][t][j] = j <= t ? pt[u] : 0.0f;                        // M[t][j]
       sTb[buf][j][t] = j > t ? pt[u] : (j == t ? 1.0f : 0.0f);       // Tinv[j][t]
     }
-    if (w == 1 && l < kC) {
-      sgb[buf][l] = pg;
-      sbb[buf][l] = pb;
-    }
   };
-  // gamma_t = e^G_t and dec_t = e^(G_31 - G_t) of a chunk, by wave 1 from the g it stashed itself
-  auto decays = [&](int buf, int db) {
-    const float Gt = prefix32(sgb[buf], l);
+  // beta, gamma_t = e^G_t and dec_t = e^(G_31 - G_t) of a chunk, by wave 1
+  auto decays = [&](int db) {
+    if (l < kC) {
+      sg[l] = pg;
+      sbb[db][l] = pb;
+    }
+    const float Gt = prefix32(sg, l);
     const float G31 = __shfl(Gt, kC - 1, 64);
     if (l < kC) {
       sgam[db][l] = q27_expf(Gt);
@@ -343,16 +357,25 @@ __global__ void __launch_bounds__(512) gdn_chunk_kernel(const float* __restrict_
   };
 
   fetch(0);
+  if (w == 1) fetch_g(0);
   stash(0);
-  if (w == 1) decays(0, 0);
+  if (w == 1) {
+    decays(0);
+    fetch_g(1);
+  }
+  fetch(1);
   __syncthreads();
 
+  // The kernel is bound by the chain of the three phases of a chunk (about 8400 cycles, 3584 of them matrix issue per
+  // SIMD), so what Delta does not need is done by the waves that wait for it: chunk ch + 1's rows go to the free buffer and
+  // chunk ch + 2's are requested beside Delta by waves 2, 3, 4, 6, 7, after the update by the Delta waves (0, 5) and wave 1,
+  // which forms the next chunk's decays beside Delta; the output tiles' gamma Q S and M operands are read there too, which
+  // leaves them 4 or 8 matrix steps in the update phase. Measured against all of it in the update phase (us, same
+  // bits): 2048 tokens 268 -> 260.6, 333 tokens 58.7 -> 56.2.
+  const bool early = !dl_wave && w != 1;
   for (int ch = 0; ch < nch; ch++) {
     const int c0 = ch * kC, n = min(kC, T - c0);
     const int rb = ch % kNB, db = ch & 1;
-    // chunk ch + 1, in flight during this chunk and stored at its end (past the last chunk: no loads, zeros into the
-    // buffer no later chunk reads; unconditional, which keeps the compiler's memory-counter waits exact)
-    fetch(ch + 1);
     // partial products X S (X = K rows or Q rows of chunk ch) over this wave's 32 state rows, into part[w][slot ..]
     auto partial = [&](const float (*X)[kKP], int slot) {
       v4f acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
@@ -372,7 +395,10 @@ __global__ void __launch_bounds__(512) gdn_chunk_kernel(const float* __restrict_
     partial(sKb[rb], 0);
     partial(sQb[rb], 2);
     __syncthreads();
-    // ---- Y: Delta = Tinv (beta (V - gamma K S)) (one wave per column half)
+    // ---- Y: Delta = Tinv (beta (V - gamma K S)) (one wave per column half); beside it the output tiles' gamma Q S and M
+    //      operands (o waves), the next chunk's rows and decays
+    v4f oz = {0.f, 0.f, 0.f, 0.f};  // the output tile (o waves)
+    float mo[8];                    // its M operands
     if (dl_wave) {
       v4f ks[2];
 #pragma unroll
@@ -388,7 +414,7 @@ __global__ void __launch_bounds__(512) gdn_chunk_kernel(const float* __restrict_
 #pragma unroll
         for (int i = 0; i < 4; i++) {
           const int t = 16 * tt + 4 * kq + i;
-          rhs[i] = sbb[rb][t] * (sVb[rb][t][16 * cb + r] - sgam[db][t] * ks[tt][i]);
+          rhs[i] = sbb[db][t] * (sVb[rb][t][16 * cb + r] - sgam[db][t] * ks[tt][i]);
         }
         rop[tt] = tile_to_operand(rhs);
       }
@@ -406,25 +432,32 @@ __global__ void __launch_bounds__(512) gdn_chunk_kernel(const float* __restrict_
         sDl[cb][4 * kq + i][r] = d0[i];
         sDl[cb][16 + 4 * kq + i][r] = d1[i];
       }
+    } else {
+      if (o_wave) {
+        v4f qs = part[4 * cb][2 + ot][l];
+#pragma unroll
+        for (int j = 1; j < 4; j++) qs += part[4 * cb + j][2 + ot][l];
+#pragma unroll
+        for (int i = 0; i < 4; i++) oz[i] = sgam[db][16 * ot + 4 * kq + i] * qs[i];
+#pragma unroll
+        for (int m = 0; m < 8; m++) mo[m] = sMb[rb][16 * ot + r][4 * m + kq];
+      }
+      if (w == 1) {
+        decays(db ^ 1);
+        fetch_g(ch + 2);
+      }
+    }
+    if (early) {
+      stash((ch + 1) % kNB);
+      fetch(ch + 2);
     }
     __syncthreads();
     // ---- Z: state update S <- gamma_31 S + sum_t dec_t k_t Delta_t^T; output tile O_ot = gamma Q S + M Delta
     //      (O_0 = gamma Q S_0 + M_00 Delta_0, O_1 = gamma Q S_1 + M_10 Delta_0 + M_11 Delta_1; Delta read from LDS
-    //      in the B-operand layout); chunk ch + 1's rows to the free buffer, its decays
-    v4f oz;  // the output tile (o waves), stored after the stash
-    if (o_wave) {
-      v4f qs = part[4 * cb][2 + ot][l];
+    //      in the B-operand layout)
+    float dl[8];
 #pragma unroll
-      for (int j = 1; j < 4; j++) qs += part[4 * cb + j][2 + ot][l];
-#pragma unroll
-      for (int i = 0; i < 4; i++) oz[i] = sgam[db][16 * ot + 4 * kq + i] * qs[i];
-#pragma unroll
-      for (int m = 0; m < 4; m++) oz = mfma4(sMb[rb][16 * ot + r][4 * m + kq], sDl[cb][4 * m + kq][r], oz);
-      if (ot == 1) {
-#pragma unroll
-        for (int m = 0; m < 4; m++) oz = mfma4(sMb[rb][16 + r][16 + 4 * m + kq], sDl[cb][16 + 4 * m + kq][r], oz);
-      }
-    }
+    for (int m = 0; m < kC / 4; m++) dl[m] = sDl[cb][4 * m + kq][r];
     {
       const float g31 = sgam[db][kC - 1];
 #pragma unroll
@@ -433,20 +466,28 @@ __global__ void __launch_bounds__(512) gdn_chunk_kernel(const float* __restrict_
 #pragma unroll
         for (int m = 0; m < kC / 4; m++) {
           const int t = 4 * m + kq;
-          S[b] = mfma4(sdec[db][t] * sKb[rb][t][32 * kb + 16 * b + r], sDl[cb][t][r], S[b]);
+          S[b] = mfma4(sdec[db][t] * sKb[rb][t][32 * kb + 16 * b + r], dl[m], S[b]);
         }
       }
     }
-    stash((ch + 1) % kNB);
-    if (w == 1) decays((ch + 1) % kNB, db ^ 1);
-    // the output stores come after the stash: vector memory counts stores and loads together, so a store issued
-    // before it would make the stash wait for the store's completion
     if (o_wave) {
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int t = 16 * ot + 4 * kq + i;
-        if (t < n) o[((size_t)(c0 + t) * H + h) * 128 + col] = oz[i] * scale;
+      for (int m = 0; m < 4; m++) oz = mfma4(mo[m], dl[m], oz);
+      if (ot == 1) {
+#pragma unroll
+        for (int m = 4; m < 8; m++) oz = mfma4(mo[m], dl[m], oz);
       }
+      const auto fo = rows_of(o + h * 128, c0, n, H * 128, 128);  // (stores past the last token are dropped)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const float x = oz[i] * scale;
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), fo,
+                                              ((16 * ot + 4 * kq + i) * H * 128 + cg * kNC + cb * 16 + r) * 4, 0, 0);
+      }
+    }
+    if (!early) {
+      stash((ch + 1) % kNB);
+      fetch(ch + 2);
     }
     __syncthreads();
   }
@@ -484,6 +525,8 @@ extern "C" int q27h_gdn_step_chunked(const float* q, const float* k, const float
   if (gdn_chunk_o_overlaps(q, k, v, stride, g, beta, planes, o, H, HK, T))
     return fail(Q27H_ERR_ARG, "gdn_step_chunked: o overlaps q / k / v rows, g, beta or the state planes");
   const hipStream_t st = stream_of(s);
+  if (!gdn_chunk_fits(stride, H))  // the sequential kernel's 64-bit offsets
+    return gdn_prefill_sequential(q, k, v, stride, g, beta, planes, in_plane, o, H, HK, T, scale, st);
   hipLaunchKernelGGL(gdn_chunk_prep_kernel, dim3(min(H, HK), (T + kC - 1) / kC), dim3(256), 0, st, q, k, stride, g, beta,
                      planes, in_plane, o, H, HK, T);
   if (int e = check_launch("gdn_step_chunked")) return e;
