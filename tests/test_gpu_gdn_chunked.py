@@ -169,6 +169,36 @@ def test_gdn_step_prefill_dispatch(q27, oracle, dev):
         q27.ops.gdn_prefill_exact(prev)
 
 
+@pytest.mark.parametrize("stride", [1 << 24, (1 << 24) + 4])
+def test_gdn_chunked_wide_rows(q27, dev, stride):
+    """Rows 2^24 floats apart (the last stride whose chunk the 32-bit offsets reach: the bits of compact rows) and
+    farther (the sequential kernel: its bits). 65 rows: a full chunk, a second one and a ragged one."""
+    import torch
+
+    H, HK, M = 2, 1, 65
+    say(f"gdn chunked stride={stride}")
+    x, W, g, beta, planes = cd.gdn_inputs(cd.rng(800), M, H, HK)
+    prev = q27.ops.gdn_prefill_exact(False)
+    try:
+        if stride <= 1 << 24:
+            want_o, want_p = _run(q27, dev, x, W, g, beta, planes, 0, H, HK, M)
+        else:
+            q27.ops.gdn_prefill_exact(True)
+            want_o, want_p = _run_step(q27, dev, x, W, g, beta, planes, 0, H, HK, M)
+    finally:
+        q27.ops.gdn_prefill_exact(prev)
+    dx = torch.empty((M - 1) * stride + W, device=dev)
+    dx.as_strided((M, W), (stride, 1)).copy_(torch.from_numpy(x).to(dev).view(M, W))
+    dp = torch.from_numpy(planes).to(dev)
+    pin = torch.zeros(1, dtype=torch.int32, device=dev)
+    o = torch.full((M * H * 128,), float("nan"), device=dev)
+    q27.ops.gdn_step_chunked(dx, dx[HK * 128:], dx[2 * HK * 128:], stride, torch.from_numpy(g).to(dev),
+                             torch.from_numpy(beta).to(dev), dp, pin, o, H, HK, M, float(SCALE))
+    torch.cuda.synchronize()
+    assert np.array_equal(o.cpu().numpy().view(np.uint32), want_o.view(np.uint32))
+    assert np.array_equal(dp.cpu().numpy().view(np.uint32), want_p.view(np.uint32))
+
+
 def test_gdn_chunked_replays_in_hip_graph(q27, dev):
     """The chunked prefill (two launches, Tinv / M staged in o) captured in a HIP graph: every replay gives the eager
     launch's bits (no allocation, no host synchronisation, nothing left over from the previous replay)."""
