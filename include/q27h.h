@@ -209,8 +209,8 @@ int q27h_qgemv(int type, int N, int K, const void* buf, const int8_t* xq, const 
  * (K * 2 for three columns), else Q27H_ERR_SHAPE. Slower than the pair at the decode shapes (every workgroup
  * quantizes the whole x): 5120 x 6144 at four columns 21-23 against 12-13 us. */
 int q27h_qgemv_f32(int type, int N, int K, const void* buf, const float* x, float* y, int ncols, q27h_stream_t s);
-/* Waves that share one 8-row tile in a q27h_qgemv launch of ncols columns (1..16; three columns run as launches of two
- * and one): part of the summation order, a function of the type, K and ncols only. */
+/* Waves that share one 8-row tile in a q27h_qgemv call of ncols columns (1..16; the sums of three columns are ordered as
+ * those of a call of two and one of one): part of the summation order, a function of the type, K and ncols only. */
 int q27h_qgemv_waves(int type, int K, int ncols);
 
 /* ---------------------------------------------------------------- GGUF reader (src/gguf.h, src/gguf.cpp)

@@ -845,8 +845,9 @@ template <int TYPE, int NC, bool NTP, bool ONE, bool FUSED = false>
 __device__ __forceinline__ void qgemv_body(Mat m, const int8_t* __restrict__ xq, const float* __restrict__ xd,
                                            float* __restrict__ y, int K, int W, const float* __restrict__ xf = nullptr) {
   constexpr int LW = LutInfo<TYPE>::words;
+  constexpr int VC = NC == 3 ? 4 : NC;  // columns of the butterfly (three: the fourth's values are the constant 0)
   __shared__ uint32_t lut[LW > 0 ? LW : 1];
-  __shared__ float part[kMaxW][8 * NC];
+  __shared__ float part[kMaxW][8 * VC];
   if constexpr (FUSED) {
     __shared__ __align__(16) int8_t s_xq[kFusedMaxX];
     __shared__ float s_xd[kFusedMaxX / 32];
@@ -955,29 +956,32 @@ __device__ __forceinline__ void qgemv_body(Mat m, const int8_t* __restrict__ xq,
       }
     }
   }
-  // 64-lane butterfly; afterwards lane l holds value index l >> (6 - log2(8 NC)) (copies in the lower lane bits)
-  constexpr int V = 8 * NC;
+  // 64-lane butterfly; afterwards lane l holds value index l >> (6 - log2(8 VC)) (copies in the lower lane bits)
+  constexpr int V = 8 * VC;
+  float red[V];
+#pragma unroll
+  for (int i = 0; i < V; i++) red[i] = i % VC < NC ? acc[i / VC * NC + i % VC] : 0.0f;
   constexpr int c1 = V, c2 = c1 > 1 ? c1 / 2 : 1, c3 = c2 > 1 ? c2 / 2 : 1, c4 = c3 > 1 ? c3 / 2 : 1,
                 c5 = c4 > 1 ? c4 / 2 : 1, c6 = c5 > 1 ? c5 / 2 : 1;
-  reduce_level<32, c1>(acc, lane);
-  reduce_level<16, c2>(acc, lane);
-  reduce_level<8, c3>(acc, lane);
-  reduce_level<4, c4>(acc, lane);
-  reduce_level<2, c5>(acc, lane);
-  reduce_level<1, c6>(acc, lane);
-  constexpr int shift = V == 8 ? 3 : V == 16 ? 2 : V == 32 ? 1 : 0;  // NC = 3 (V = 24) is handled on the host
+  reduce_level<32, c1>(red, lane);
+  reduce_level<16, c2>(red, lane);
+  reduce_level<8, c3>(red, lane);
+  reduce_level<4, c4>(red, lane);
+  reduce_level<2, c5>(red, lane);
+  reduce_level<1, c6>(red, lane);
+  constexpr int shift = V == 8 ? 3 : V == 16 ? 2 : 1;
   const int idx = lane >> shift;
-  const bool writer = (lane & ((1 << shift) - 1)) == 0;
+  const bool writer = (lane & ((1 << shift) - 1)) == 0 && idx % VC < NC;
   if (W == 1) {
-    if (live && writer) y[(size_t)(idx % NC) * m.N + tile * 8 + idx / NC] = acc[0];
+    if (live && writer) y[(size_t)(idx % VC) * m.N + tile * 8 + idx / VC] = red[0];
     return;
   }
-  if (writer) part[wave][idx] = acc[0];
+  if (writer) part[wave][idx] = red[0];
   __syncthreads();
   if (live && wv == 0 && writer) {
     float t = part[wave][idx];
     for (int k = 1; k < W; k++) t = t + part[wave + k][idx];
-    y[(size_t)(idx % NC) * m.N + tile * 8 + idx / NC] = t;
+    y[(size_t)(idx % VC) * m.N + tile * 8 + idx / VC] = t;
   }
 }
 
@@ -990,20 +994,32 @@ __device__ __forceinline__ void qgemv_body(Mat m, const int8_t* __restrict__ xq,
 // 13.7 -> 14.3 us), the opposite of the prefetching kernel.
 // IQ3_S with four columns needed a few more than 128 VGPRs here and spilled 12 bytes per lane to scratch (about 2 MB
 // of scratch traffic per 17408 x 5120 launch) until the sums of half the rows were parked in LDS (parks_sums).
-#ifndef Q27H_QG_WPE_ONE
-#define Q27H_QG_WPE_ONE 4
-#endif
+// Three columns: 6 waves per SIMD (80 VGPRs) instead of 4 also let two workgroups of nine waves (K = 17408) share a CU
+// (us, 17408 x 5120 / 5120 x 17408, 4 -> 6: Q4_K 16.3 / 22.7 -> 14.4 / 16.1, IQ2_XS 20.1 / 25.6 -> 17.1 / 18.5, IQ4_XS
+// 18.3 / 22.3 -> 15.9 / 17.8); Q6_K spills at 6 (27.3 / 28.8, at 5 18.3 / 24.7), IQ3_XXS and IQ3_S run slower (16.4 and
+// 16.5, at 5 15.5 and 15.6).
+constexpr int one_waves_per_simd(int type, int nc) {
+  if (nc == 3) return type == kQ6K || type == kIQ3XXS || type == kIQ3S ? 5 : 6;
+  return 4;
+}
 template <int TYPE, int NC, bool NTP, bool FUSED = false>
 __global__ void __launch_bounds__(256) qgemv_kernel(Mat m, const int8_t* __restrict__ xq, const float* __restrict__ xd,
                                                     float* __restrict__ y, int K, int W, const float* __restrict__ xf) {
   qgemv_body<TYPE, NC, NTP, false, FUSED>(m, xq, xd, y, K, W, xf);
 }
 template <int TYPE, int NC, bool FUSED = false>
-__global__ void __launch_bounds__(64 * kMaxW) __attribute__((amdgpu_waves_per_eu(Q27H_QG_WPE_ONE)))
+__global__ void __launch_bounds__(64 * kMaxW) __attribute__((amdgpu_waves_per_eu(one_waves_per_simd(TYPE, NC))))
 qgemv_one_kernel(Mat m, const int8_t* __restrict__ xq, const float* __restrict__ xd, float* __restrict__ y, int K, int W,
                  const float* __restrict__ xf) {
   qgemv_body<TYPE, NC, true, true, FUSED>(m, xq, xd, y, K, W, xf);
 }
+
+// Three columns: the order of the sums is that of two columns, then one. Where both take the same waves (all but
+// IQ3_XXS / IQ3_S / IQ1_M at 8192 < K <= 32768) one launch gives the same bits and reads and decodes the weights once.
+// Measured against two launches (us, 17408 x 5120 / 5120 x 17408): Q4_K 22.1 -> 14.4 / 23.4 -> 16.1, Q6_K 28.9 -> 18.3 /
+// 30.5 -> 24.7, IQ2_XS 23.9 -> 17.1 / 22.9 -> 18.5, IQ4_XS 24.7 -> 15.9 / 25.7 -> 17.8, IQ3_S 26.6 -> 15.6, IQ1_M 27.5 ->
+// 21.6; smaller matrices (1024 x 5120, 2048 x 1024) 1.4-1.7 times as fast.
+constexpr bool three_in_one(int type, int K) { return waves_per_tile(type, K, 2) == waves_per_tile(type, K, 1); }
 
 int check_type(int type) {
   if (fmt_of(type).nf == 0) return fail(Q27H_ERR_UNSUPPORTED, "qgemv: weight type " + std::to_string(type) + " not supported");
@@ -1012,7 +1028,7 @@ int check_type(int type) {
 
 template <int TYPE, int NC, bool FUSED = false>
 void launch_gemv(const Mat& m, const int8_t* xq, const float* xd, float* y, int K, hipStream_t s, const float* xf = nullptr) {
-  const int W = waves_per_tile(TYPE, K, NC);
+  const int W = waves_per_tile(TYPE, K, NC == 3 ? 1 : NC);
   const int grid = m.ntiles;
   // the prefetching kernel takes at most 4 waves (lanes with several blocks); W > 4 means one block per lane
   const bool one = m.nb <= 8 * W && (W > 4 || !((TYPE == kQ2K || TYPE == kQ4K) && NC == 4));
@@ -1029,6 +1045,7 @@ void launch_nc(const Mat& m, const int8_t* xq, const float* xd, float* y, int K,
                const float* xf = nullptr) {
   if (nc == 1) launch_gemv<TYPE, 1, FUSED>(m, xq, xd, y, K, s, xf);
   else if (nc == 2) launch_gemv<TYPE, 2, FUSED>(m, xq, xd, y, K, s, xf);
+  else if (nc == 3) launch_gemv<TYPE, 3, FUSED>(m, xq, xd, y, K, s, xf);
   else launch_gemv<TYPE, 4, FUSED>(m, xq, xd, y, K, s, xf);
 }
 
@@ -1088,7 +1105,7 @@ extern "C" int q27h_qgemv(int type, int N, int K, const void* buf, const int8_t*
   const uint8_t* b = (const uint8_t*)buf;
   const Mat m{{b + off[0], b + off[1], b + off[2], b + off[3]}, b + off[4], N, K / 256, N / 8};
   const hipStream_t st = stream_of(s);
-  // three columns run as two launches (columns 0-1, then column 2), each with its own rows of y
+  // three columns whose one- and two-column sums take different waves run as two launches (columns 0-1, then column 2)
   auto run = [&](const int8_t* q, const float* d, float* yy, int nc) {
     switch (type) {
       case kQ2K: launch_nc<kQ2K>(m, q, d, yy, K, nc, st); break;
@@ -1103,7 +1120,7 @@ extern "C" int q27h_qgemv(int type, int N, int K, const void* buf, const int8_t*
       default: launch_nc<kIQ4XS>(m, q, d, yy, K, nc, st); break;
     }
   };
-  if (ncols == 3) {
+  if (ncols == 3 && !three_in_one(type, K)) {
     run(xq, xd, y, 2);
     run(xq + (size_t)2 * K, xd + (size_t)2 * (K / 32), y + (size_t)2 * N, 1);
   } else {
@@ -1140,7 +1157,7 @@ extern "C" int q27h_qgemv_f32(int type, int N, int K, const void* buf, const flo
       default: launch_nc<kIQ4XS, true>(m, nullptr, nullptr, yy, K, nc, st, xx); break;
     }
   };
-  if (ncols == 3) {
+  if (ncols == 3 && !(three_in_one(type, K) && (long)K * 3 <= kFusedMaxX)) {
     run(x, y, 2);
     run(x + (size_t)2 * K, y + (size_t)2 * N, 1);
   } else {

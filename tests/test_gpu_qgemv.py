@@ -71,6 +71,32 @@ def test_qgemv_columns_wide_k(q27, oracle, dev, type_, ncols):
         assert_bits_equal(got, want, f"qgemv type {type_} {N}x{K} ncols {ncols}")
 
 
+@pytest.mark.parametrize("type_", TYPES)
+@pytest.mark.parametrize("N,K,f32", [(8, 256, False), (24, 8192, False), (24, 8448, False), (24, 32768, False),
+                                     (24, 33024, False), (8, 13568, True), (8, 13824, True)])
+def test_qgemv_three_columns(q27, oracle, dev, type_, N, K, f32):
+    """Where three columns change between one launch and two: the last K at which IQ3_XXS / IQ3_S / IQ1_M take the same
+    waves for one and two columns and the next, the last K with one block per lane and the next (prefetching kernel);
+    f32 activations: the last K whose three columns fit in LDS and the next."""
+    import torch
+
+    say(f"qgemv three columns type {type_} {N}x{K} f32={f32}")
+    r = cd.rng(480 + type_ + K)
+    raw = cd.random_weights(r, type_, N, K)
+    if f32:
+        x = r.standard_normal(3 * K).astype(np.float32)
+        m = q27.ops.qmat_upload(torch.from_numpy(raw).to(dev), type_, N, K)
+        y = torch.full((3 * N,), float("nan"), device=dev)
+        q27.ops.qgemv_f32(m, torch.from_numpy(x).to(dev), y, 3)
+        got = y.cpu().numpy().reshape(3, N)
+        xq, xd, _ = oracle.quantize_q8_1(x, K, 3)
+    else:
+        xq, xd = cd.q8_activations(oracle, r, 3, K)
+        got = _run(q27, dev, type_, N, K, raw, xq, xd, 3)
+    want = oracle.qgemv(type_, raw, N, K, xq, xd, 3)
+    assert_bits_equal(got, np.asarray(want).reshape(3, N), f"qgemv three columns type {type_} {N}x{K}")
+
+
 def test_qgemv_small_and_edge_shapes(q27, oracle, dev):
     """One tile, one block per row, and partial 8-block groups; zero activations and wide scale ranges."""
     for type_ in TYPES:
