@@ -841,7 +841,11 @@ constexpr int waves_per_tile(int type, int K, int ncols) {
 // code of quantize_q8_1 (q8_1_store_n: amax, d = amax / 127, q = roundf(y / d), scale fp16(d)), then reads them from
 // there. The results are those of quantize_q8_1 followed by the unfused GEMV, bit for bit.
 constexpr int kFusedMaxX = 40960;  // NC * K values a fused launch may quantize per workgroup (40 KB of int8 in LDS)
-template <int TYPE, int NC, bool NTP, bool ONE, bool FUSED = false>
+// FOLD: every wave of the workgroup takes one block per lane as in ONE, but the sums are those of W waves whose lanes
+// take several blocks: before the butterfly the waves W, W + 1, ... hand their lanes' sums over in LDS, and wave w adds
+// those of w + W, w + 2 W, ... in order (a lane without a block has +0). Of three columns the third is ordered by one
+// block per lane, so its sums stay where they are.
+template <int TYPE, int NC, bool NTP, bool ONE, bool FUSED = false, bool FOLD = false>
 __device__ __forceinline__ void qgemv_body(Mat m, const int8_t* __restrict__ xq, const float* __restrict__ xd,
                                            float* __restrict__ y, int K, int W, const float* __restrict__ xf = nullptr) {
   constexpr int LW = LutInfo<TYPE>::words;
@@ -956,6 +960,23 @@ __device__ __forceinline__ void qgemv_body(Mat m, const int8_t* __restrict__ xq,
       }
     }
   }
+  const int nw = FOLD ? (int)(blockDim.x >> 6) : W;
+  if constexpr (FOLD) {
+    extern __shared__ float fold[];
+    constexpr int FC = NC == 3 ? 2 : NC;
+    if (wave >= W) {
+      float* f = fold + (wave - W) * (8 * FC * 64) + lane;
+#pragma unroll
+      for (int i = 0; i < 8 * FC; i++) f[i * 64] = acc[i / FC * NC + i % FC];
+    }
+    __syncthreads();
+    if (wave < W)
+      for (int p = wave; p + W < nw; p += W) {
+        const float* f = fold + p * (8 * FC * 64) + lane;
+#pragma unroll
+        for (int i = 0; i < 8 * FC; i++) acc[i / FC * NC + i % FC] += f[i * 64];
+      }
+  }
   // 64-lane butterfly; afterwards lane l holds value index l >> (6 - log2(8 VC)) (copies in the lower lane bits)
   constexpr int V = 8 * VC;
   float red[V];
@@ -980,11 +1001,19 @@ __device__ __forceinline__ void qgemv_body(Mat m, const int8_t* __restrict__ xq,
   __syncthreads();
   if (live && wv == 0 && writer) {
     float t = part[wave][idx];
-    for (int k = 1; k < W; k++) t = t + part[wave + k][idx];
+    const int n = NC == 3 && idx % VC == 2 ? nw : W;
+    for (int k = 1; k < n; k++) t = t + part[wave + k][idx];
     y[(size_t)(idx % VC) * m.N + tile * 8 + idx / VC] = t;
   }
 }
 
+// IQ3_XXS / IQ3_S / IQ1_M, two or three columns, 8192 < K <= 32768: 4 waves' sums formed by one block per lane. Three
+// columns ran as launches of two and one, two on the prefetching kernel. Measured (us, 5120 x 17408 / 5120 x 10240 / 1024 x
+// 20480): T = 3 IQ3_S 27.3 / 19.6 / 15.8 -> 19.2 / 12.2 / 9.6, IQ3_XXS 26.4 / 18.7 / 16.2 -> 19.0 / 12.0 / 9.5, IQ1_M 28.8 /
+// 20.7 / 17.4 -> 28.8 / 14.4 / 11.5; T = 2 IQ3_S 17.4 / 12.0 / 9.6 -> 17.5 / 10.8 / 8.4, IQ3_XXS 16.9 / 11.6 / 10.3 -> 16.4 /
+// 10.2 / 8.1, IQ1_M 18.8 / 13.3 / 11.3 -> 16.9 / 11.1 / 8.7. Four columns ran slower (5120 x 17408 Q4_K 18.6 -> 24-26, IQ3_S
+// 20.9 -> 27.7: 9 waves of 96 VGPRs and 40 KB per workgroup, 640 workgroups are 1.25 rounds of the CUs).
+constexpr bool folds(int type, int nc) { return (nc == 2 || nc == 3) && (type == kIQ3XXS || type == kIQ3S || type == kIQ1M); }
 // Kernel for K <= 2048 W (every lane takes at most one block of its tile): no prefetch registers, and the compiler is
 // held to 128 VGPRs (4 waves per SIMD) for four columns. Measured against the prefetching kernel (us, 17408 x 5120,
 // T = 1 / T = 4): Q4_K 10.9 -> 9.8 / 17.3 -> 17.9, Q6_K 14.7 -> 13.1 / 20.0 -> 19.3, IQ3_S 13.2 -> 11.4 / 20.3 -> 19.3,
@@ -994,12 +1023,20 @@ __device__ __forceinline__ void qgemv_body(Mat m, const int8_t* __restrict__ xq,
 // 13.7 -> 14.3 us), the opposite of the prefetching kernel.
 // IQ3_S with four columns needed a few more than 128 VGPRs here and spilled 12 bytes per lane to scratch (about 2 MB
 // of scratch traffic per 17408 x 5120 launch) until the sums of half the rows were parked in LDS (parks_sums).
-// Three columns: 6 waves per SIMD (80 VGPRs) instead of 4 also let two workgroups of nine waves (K = 17408) share a CU
+// Four columns are held to 128 VGPRs (4 waves per SIMD; IQ2_S to 96: 17408 x 5120 24.4 -> 23.1 us, the other types are
+// slower or the same). Two columns: 80 VGPRs where the compiler took more (17408 x 5120: IQ3_XXS 15.4 -> 12.8, IQ3_S
+// 15.8 -> 13.4, IQ1_M 17.1 -> 15.0).
+// Three columns in one launch (two launches before: every weight read and decoded twice), us, 17408 x 5120 / 5120 x 17408:
+// Q4_K 22.1 -> 14.4 / 23.4 -> 16.1, Q6_K 28.9 -> 18.3 / 30.5 -> 24.7, IQ2_XS 23.9 -> 17.1 / 22.9 -> 18.5, IQ4_XS 24.7 ->
+// 15.9 / 25.7 -> 17.8, IQ3_S 26.6 -> 15.6, IQ1_M 27.5 -> 21.6; smaller matrices (1024 x 5120, 2048 x 1024) 1.4-1.7 times as
+// fast. 6 waves per SIMD (80 VGPRs) instead of 4 also let two workgroups of nine waves (K = 17408) share a CU
 // (us, 17408 x 5120 / 5120 x 17408, 4 -> 6: Q4_K 16.3 / 22.7 -> 14.4 / 16.1, IQ2_XS 20.1 / 25.6 -> 17.1 / 18.5, IQ4_XS
 // 18.3 / 22.3 -> 15.9 / 17.8); Q6_K spills at 6 (27.3 / 28.8, at 5 18.3 / 24.7), IQ3_XXS and IQ3_S run slower (16.4 and
 // 16.5, at 5 15.5 and 15.6).
 constexpr int one_waves_per_simd(int type, int nc) {
   if (nc == 3) return type == kQ6K || type == kIQ3XXS || type == kIQ3S ? 5 : 6;
+  if (nc == 2) return folds(type, 2) ? 6 : 4;
+  if (nc == 4) return type == kIQ2S ? 5 : 4;
   return 4;
 }
 template <int TYPE, int NC, bool NTP, bool FUSED = false>
@@ -1014,12 +1051,14 @@ qgemv_one_kernel(Mat m, const int8_t* __restrict__ xq, const float* __restrict__
   qgemv_body<TYPE, NC, true, true, FUSED>(m, xq, xd, y, K, W, xf);
 }
 
-// Three columns: the order of the sums is that of two columns, then one. Where both take the same waves (all but
-// IQ3_XXS / IQ3_S / IQ1_M at 8192 < K <= 32768) one launch gives the same bits and reads and decodes the weights once.
-// Measured against two launches (us, 17408 x 5120 / 5120 x 17408): Q4_K 22.1 -> 14.4 / 23.4 -> 16.1, Q6_K 28.9 -> 18.3 /
-// 30.5 -> 24.7, IQ2_XS 23.9 -> 17.1 / 22.9 -> 18.5, IQ4_XS 24.7 -> 15.9 / 25.7 -> 17.8, IQ3_S 26.6 -> 15.6, IQ1_M 27.5 ->
-// 21.6; smaller matrices (1024 x 5120, 2048 x 1024) 1.4-1.7 times as fast.
-constexpr bool three_in_one(int type, int K) { return waves_per_tile(type, K, 2) == waves_per_tile(type, K, 1); }
+// Three columns: the order of the sums is that of two columns, then that of one. Whether both take the same waves (all but
+// IQ3_XXS / IQ3_S / IQ1_M at 8192 < K <= 32768, which need the folding kernel).
+constexpr bool three_alike(int type, int K) { return waves_per_tile(type, K, 2) == waves_per_tile(type, K, 1); }
+template <int TYPE, int NC>
+__global__ void __launch_bounds__(64 * kMaxW) __attribute__((amdgpu_waves_per_eu(NC == 3 ? 5 : 6)))
+qgemv_fold_kernel(Mat m, const int8_t* __restrict__ xq, const float* __restrict__ xd, float* __restrict__ y, int K, int W) {
+  qgemv_body<TYPE, NC, true, true, false, true>(m, xq, xd, y, K, W);
+}
 
 int check_type(int type) {
   if (fmt_of(type).nf == 0) return fail(Q27H_ERR_UNSUPPORTED, "qgemv: weight type " + std::to_string(type) + " not supported");
@@ -1028,10 +1067,17 @@ int check_type(int type) {
 
 template <int TYPE, int NC, bool FUSED = false>
 void launch_gemv(const Mat& m, const int8_t* xq, const float* xd, float* y, int K, hipStream_t s, const float* xf = nullptr) {
-  const int W = waves_per_tile(TYPE, K, NC == 3 ? 1 : NC);
+  const int W = waves_per_tile(TYPE, K, NC == 3 ? 2 : NC);
   const int grid = m.ntiles;
   // the prefetching kernel takes at most 4 waves (lanes with several blocks); W > 4 means one block per lane
   const bool one = m.nb <= 8 * W && (W > 4 || !((TYPE == kQ2K || TYPE == kQ4K) && NC == 4));
+  if constexpr (!FUSED && folds(TYPE, NC)) {
+    const int g = (m.nb + 7) / 8;
+    if (g > W && g <= kMaxW) {
+      hipLaunchKernelGGL((qgemv_fold_kernel<TYPE, NC>), dim3(grid), dim3(64 * g), (g - W) * 16 * 256, s, m, xq, xd, y, K, W);
+      return;
+    }
+  }
   if (one)
     hipLaunchKernelGGL((qgemv_one_kernel<TYPE, NC, FUSED>), dim3(grid), dim3(64 * W), 0, s, m, xq, xd, y, K, W, xf);
   else if (K <= kNtPiecesMaxK)
@@ -1105,26 +1151,17 @@ extern "C" int q27h_qgemv(int type, int N, int K, const void* buf, const int8_t*
   const uint8_t* b = (const uint8_t*)buf;
   const Mat m{{b + off[0], b + off[1], b + off[2], b + off[3]}, b + off[4], N, K / 256, N / 8};
   const hipStream_t st = stream_of(s);
-  // three columns whose one- and two-column sums take different waves run as two launches (columns 0-1, then column 2)
-  auto run = [&](const int8_t* q, const float* d, float* yy, int nc) {
-    switch (type) {
-      case kQ2K: launch_nc<kQ2K>(m, q, d, yy, K, nc, st); break;
-      case kQ4K: launch_nc<kQ4K>(m, q, d, yy, K, nc, st); break;
-      case kQ6K: launch_nc<kQ6K>(m, q, d, yy, K, nc, st); break;
-      case kIQ2XXS: launch_nc<kIQ2XXS>(m, q, d, yy, K, nc, st); break;
-      case kIQ2XS: launch_nc<kIQ2XS>(m, q, d, yy, K, nc, st); break;
-      case kIQ3XXS: launch_nc<kIQ3XXS>(m, q, d, yy, K, nc, st); break;
-      case kIQ3S: launch_nc<kIQ3S>(m, q, d, yy, K, nc, st); break;
-      case kIQ2S: launch_nc<kIQ2S>(m, q, d, yy, K, nc, st); break;
-      case kIQ1M: launch_nc<kIQ1M>(m, q, d, yy, K, nc, st); break;
-      default: launch_nc<kIQ4XS>(m, q, d, yy, K, nc, st); break;
-    }
-  };
-  if (ncols == 3 && !three_in_one(type, K)) {
-    run(xq, xd, y, 2);
-    run(xq + (size_t)2 * K, xd + (size_t)2 * (K / 32), y + (size_t)2 * N, 1);
-  } else {
-    run(xq, xd, y, ncols);
+  switch (type) {
+    case kQ2K: launch_nc<kQ2K>(m, xq, xd, y, K, ncols, st); break;
+    case kQ4K: launch_nc<kQ4K>(m, xq, xd, y, K, ncols, st); break;
+    case kQ6K: launch_nc<kQ6K>(m, xq, xd, y, K, ncols, st); break;
+    case kIQ2XXS: launch_nc<kIQ2XXS>(m, xq, xd, y, K, ncols, st); break;
+    case kIQ2XS: launch_nc<kIQ2XS>(m, xq, xd, y, K, ncols, st); break;
+    case kIQ3XXS: launch_nc<kIQ3XXS>(m, xq, xd, y, K, ncols, st); break;
+    case kIQ3S: launch_nc<kIQ3S>(m, xq, xd, y, K, ncols, st); break;
+    case kIQ2S: launch_nc<kIQ2S>(m, xq, xd, y, K, ncols, st); break;
+    case kIQ1M: launch_nc<kIQ1M>(m, xq, xd, y, K, ncols, st); break;
+    default: launch_nc<kIQ4XS>(m, xq, xd, y, K, ncols, st); break;
   }
   return check_launch("qgemv");
 }
@@ -1157,7 +1194,7 @@ extern "C" int q27h_qgemv_f32(int type, int N, int K, const void* buf, const flo
       default: launch_nc<kIQ4XS, true>(m, nullptr, nullptr, yy, K, nc, st, xx); break;
     }
   };
-  if (ncols == 3 && !(three_in_one(type, K) && (long)K * 3 <= kFusedMaxX)) {
+  if (ncols == 3 && !(three_alike(type, K) && (long)K * 3 <= kFusedMaxX)) {
     run(x, y, 2);
     run(x + (size_t)2 * K, y + (size_t)2 * N, 1);
   } else {
