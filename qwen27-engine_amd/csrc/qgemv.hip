@@ -21,22 +21,22 @@ namespace {
 constexpr int kQ2K = 10, kQ4K = 12, kQ6K = 14, kIQ2XXS = 16, kIQ2XS = 17, kIQ3XXS = 18, kIQ3S = 21, kIQ2S = 22,
               kIQ4XS = 23, kIQ1M = 29;
 
-__device__ const uint32_t kIQ3SGrid[512] = {
+__device__ const __align__(16) uint32_t kIQ3SGrid[512] = {
 #include "iq3s_grid.inc"
 };
-__device__ const uint32_t kIQ3XXSGrid[256] = {
+__device__ const __align__(16) uint32_t kIQ3XXSGrid[256] = {
 #include "iq3xxs_grid.inc"
 };
-__device__ const uint64_t kIQ2XXSGrid[256] = {
+__device__ const __align__(16) uint64_t kIQ2XXSGrid[256] = {
 #include "iq2xxs_grid.inc"
 };
-__device__ const uint64_t kIQ2XSGrid[512] = {
+__device__ const __align__(16) uint64_t kIQ2XSGrid[512] = {
 #include "iq2xs_grid.inc"
 };
-__device__ const uint64_t kIQ2SGrid[1024] = {
+__device__ const __align__(16) uint64_t kIQ2SGrid[1024] = {
 #include "iq2s_grid.inc"
 };
-__device__ const uint32_t kIQ1SGrid[2048] = {
+__device__ const __align__(16) uint32_t kIQ1SGrid[2048] = {
 #include "iq1s_grid.inc"
 };
 __device__ const int8_t kIQ4NL[16] = {
@@ -408,6 +408,17 @@ struct LutInfo {
   static constexpr int masks = TYPE == kIQ3S || TYPE == kIQ2S ? 256 : TYPE == kIQ2XXS || TYPE == kIQ2XS || TYPE == kIQ3XXS ? 128 : 0;
   static constexpr int words = grid + 2 * masks;
 };
+
+// The codebook as it lies in LDS: `grid` words (the 8-byte entries of the IQ2 types low word first).
+template <int TYPE>
+__device__ __forceinline__ const void* grid_of() {
+  if constexpr (TYPE == kIQ3S) return kIQ3SGrid;
+  else if constexpr (TYPE == kIQ3XXS) return kIQ3XXSGrid;
+  else if constexpr (TYPE == kIQ1M) return kIQ1SGrid;
+  else if constexpr (TYPE == kIQ2XXS) return kIQ2XXSGrid;
+  else if constexpr (TYPE == kIQ2XS) return kIQ2XSGrid;
+  else return kIQ2SGrid;
+}
 
 template <int TYPE>
 struct Chunk {
@@ -804,6 +815,12 @@ __device__ __forceinline__ float xchg(float v) {
   if constexpr (O == 32) return lane_xor32(v);
   else return lane_xor<O>(v);
 }
+// The three-column kernel reduces a padded copy of its sums, the others their sums in place.
+template <bool FIRST, class A, class B>
+__device__ __forceinline__ auto& pick(A& a, B& b) {
+  if constexpr (FIRST) return a;
+  else return b;
+}
 // One butterfly level over the first CUR live values: lanes with bit O set keep the upper half, the others the lower
 // half; each adds the partner's copy of the same values. The two candidates are chosen with bit masks (v_bfi), so no
 // value is ever selected by a per-lane index (which the compiler would lower to a compare chain over all values).
@@ -850,7 +867,7 @@ __device__ __forceinline__ void qgemv_body(Mat m, const int8_t* __restrict__ xq,
                                            float* __restrict__ y, int K, int W, const float* __restrict__ xf = nullptr) {
   constexpr int LW = LutInfo<TYPE>::words;
   constexpr int VC = NC == 3 ? 4 : NC;  // columns of the butterfly (three: the fourth's values are the constant 0)
-  __shared__ uint32_t lut[LW > 0 ? LW : 1];
+  __shared__ __align__(16) uint32_t lut[LW > 0 ? LW : 1];
   __shared__ float part[kMaxW][8 * VC];
   if constexpr (FUSED) {
     __shared__ __align__(16) int8_t s_xq[kFusedMaxX];
@@ -869,25 +886,17 @@ __device__ __forceinline__ void qgemv_body(Mat m, const int8_t* __restrict__ xq,
   }
   if constexpr (LW > 0) {
     constexpr int G = LutInfo<TYPE>::grid, NM = LutInfo<TYPE>::masks;
-    for (int i = threadIdx.x; i < G; i += blockDim.x) {
-      uint32_t v;
-      if constexpr (TYPE == kIQ3S) v = kIQ3SGrid[i];
-      else if constexpr (TYPE == kIQ3XXS) v = kIQ3XXSGrid[i];
-      else if constexpr (TYPE == kIQ1M) v = kIQ1SGrid[i];
-      else if constexpr (TYPE == kIQ2XXS) v = (uint32_t)(kIQ2XXSGrid[i / 2] >> (32 * (i & 1)));
-      else if constexpr (TYPE == kIQ2XS) v = (uint32_t)(kIQ2XSGrid[i / 2] >> (32 * (i & 1)));
-      else v = (uint32_t)(kIQ2SGrid[i / 2] >> (32 * (i & 1)));
-      lut[i] = v;
-    }
+    // Every workgroup fills its tables before its first weight, so this is latency on every launch: 16-byte pieces of the
+    // codebook and a mask pair in a few operations instead of 4-byte pieces and a loop over the bits (us, T = 1: 1024 x
+    // 5120 IQ2_S 5.3 -> 4.4, IQ1_M 4.8 -> 3.9, IQ3_S 4.4 -> 4.1; 17408 x 5120 IQ2_S 12.7 -> 11.2, IQ2_XS 11.3 -> 10.4, IQ3_S
+    // 12.5 -> 12.2; 32768 x 512 IQ2_S 15.9 -> 9.9). Requesting the weights or activations before the tables measured slower
+    // at T = 1 (17408 x 5120 IQ3_S 13.3): a workgroup's weights then wait for the whole fill in registers.
+    for (int i = threadIdx.x; i < G / 4; i += blockDim.x) ((u32x4*)lut)[i] = ((const u32x4*)grid_of<TYPE>())[i];
     for (int i = threadIdx.x; i < NM; i += blockDim.x) {
-      const int sb = NM == 128 ? (i | ((__builtin_popcount(i) & 1) << 7)) : i;  // ksigns: even count of negatives
-      uint32_t m0 = 0, m1 = 0;
-      for (int j = 0; j < 4; j++) {
-        m0 |= ((sb >> j) & 1) ? 0xFFu << (8 * j) : 0u;
-        m1 |= ((sb >> (4 + j)) & 1) ? 0xFFu << (8 * j) : 0u;
-      }
-      lut[G + 2 * i] = m0;
-      lut[G + 2 * i + 1] = m1;
+      const uint32_t sb = NM == 128 ? (i | ((__builtin_popcount(i) & 1) << 7)) : i;  // ksigns: even count of negatives
+      // bit j of a nibble to bit 8 j, then each byte 0x00 or 0xFF
+      lut[G + 2 * i] = (((sb & 0xF) * 0x204081u) & 0x01010101u) * 0xFFu;
+      lut[G + 2 * i + 1] = (((sb >> 4) * 0x204081u) & 0x01010101u) * 0xFFu;
     }
   }
   uint32_t kv[4] = {0, 0, 0, 0};
@@ -979,9 +988,12 @@ __device__ __forceinline__ void qgemv_body(Mat m, const int8_t* __restrict__ xq,
   }
   // 64-lane butterfly; afterwards lane l holds value index l >> (6 - log2(8 VC)) (copies in the lower lane bits)
   constexpr int V = 8 * VC;
-  float red[V];
+  float padded[NC == 3 ? V : 1];
+  if constexpr (NC == 3) {
 #pragma unroll
-  for (int i = 0; i < V; i++) red[i] = i % VC < NC ? acc[i / VC * NC + i % VC] : 0.0f;
+    for (int i = 0; i < V; i++) padded[i] = i % VC < NC ? acc[i / VC * NC + i % VC] : 0.0f;
+  }
+  float(&red)[V] = pick<NC == 3>(padded, acc);
   constexpr int c1 = V, c2 = c1 > 1 ? c1 / 2 : 1, c3 = c2 > 1 ? c2 / 2 : 1, c4 = c3 > 1 ? c3 / 2 : 1,
                 c5 = c4 > 1 ? c4 / 2 : 1, c6 = c5 > 1 ? c5 / 2 : 1;
   reduce_level<32, c1>(red, lane);
