@@ -143,6 +143,11 @@ __device__ __forceinline__ v4f unit_lower_inverse(const float (*B)[kPP], int r, 
 // (16 key heads x 64 chunks) is resident at once: 25.4 us against 31.5 us at three per CU, where the grid ran as two
 // successive waves of workgroups. The kernel moves 84 MB (k and q rows in, four copies of P out), about 14 us of HBM
 // time.
+// A workgroup's own chain (rows 6000 cycles, grams 3000-4800, 7400 per value head) is the whole launch when few chunks are
+// there, so up to kPrepResident workgroups (all resident: four on each of 256 CUs) every value head gets a workgroup of
+// its own, which forms the grams again. gdn_step in us, 48 value heads on 16 key heads: 128 tokens 30.9 -> 26.8, 333 56.2 ->
+// 54.6; where it lies: 700 tokens (1056 workgroups) 99.5 unsplit, 99.4 split, 1000 137.2 and 140.2, 2048 262 and 277.
+constexpr int kPrepResident = 1024;
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 gdn_chunk_prep_kernel(const float* __restrict__ q, const float* __restrict__ k, int stride, const float* __restrict__ g,
                       const float* __restrict__ beta, float* __restrict__ planes, const int* __restrict__ in_plane,
@@ -158,6 +163,7 @@ gdn_chunk_prep_kernel(const float* __restrict__ q, const float* __restrict__ k, 
   float(*sX)[kPP] = (float(*)[kPP])(smem + kC * kPP);
   float(*sP)[kPP] = (float(*)[kPP])(smem + 2 * kC * kPP);
   const int kh = blockIdx.x, c = blockIdx.y;
+  const int h0 = kh + HK * blockIdx.z, step = HK * gridDim.z;  // this workgroup's value heads
   const int c0 = c * kC, n = min(kC, T - c0);
   const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, r = l & 15, kq = l >> 4;
   // g and beta of value head hh (wave 0, one token per lane), loaded a value head ahead of their use
@@ -168,7 +174,7 @@ gdn_chunk_prep_kernel(const float* __restrict__ q, const float* __restrict__ k, 
       pb = hh < H && l < n ? beta[(size_t)(c0 + l) * H + hh] : 0.0f;
     }
   };
-  fetch_gb(kh);
+  fetch_gb(h0);
 #pragma unroll
   for (int j = 0; j < 4; j++) {
     const int e = tid + 256 * j, t = e >> 5, e4 = (e & 31) * 4;
@@ -190,12 +196,12 @@ gdn_chunk_prep_kernel(const float* __restrict__ q, const float* __restrict__ k, 
   }
   const size_t plane_sz = (size_t)H * 128 * 128;
   const int pout = *in_plane == 0 ? 1 : 0;
-  for (int h = kh; h < H; h += HK) {
+  for (int h = h0; h < H; h += step) {
     if (w == 0 && l < kC) {
       sg[l] = pg;
       sb[l] = pb;
     }
-    fetch_gb(h + HK);
+    fetch_gb(h + step);
     __syncthreads();  // also: every wave's gram reads of the k / q rows are done before -A overwrites them
     if (w < 3) {
       const float Gt = prefix32(sg, l);
@@ -527,7 +533,9 @@ extern "C" int q27h_gdn_step_chunked(const float* q, const float* k, const float
   const hipStream_t st = stream_of(s);
   if (!gdn_chunk_fits(stride, H))  // the sequential kernel's 64-bit offsets
     return gdn_prefill_sequential(q, k, v, stride, g, beta, planes, in_plane, o, H, HK, T, scale, st);
-  hipLaunchKernelGGL(gdn_chunk_prep_kernel, dim3(min(H, HK), (T + kC - 1) / kC), dim3(256), 0, st, q, k, stride, g, beta,
+  const int keys = min(H, HK), chunks = (T + kC - 1) / kC, heads = (H + HK - 1) / HK;
+  const int split = (long)keys * chunks * heads <= kPrepResident ? heads : 1;
+  hipLaunchKernelGGL(gdn_chunk_prep_kernel, dim3(keys, chunks, split), dim3(256), 0, st, q, k, stride, g, beta,
                      planes, in_plane, o, H, HK, T);
   if (int e = check_launch("gdn_step_chunked")) return e;
   hipLaunchKernelGGL(gdn_chunk_kernel, dim3(H, 128 / kNC), dim3(512), 0, st, q, k, v, stride, g, beta, planes, in_plane,

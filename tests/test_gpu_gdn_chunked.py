@@ -169,6 +169,19 @@ def test_gdn_step_prefill_dispatch(q27, oracle, dev):
         q27.ops.gdn_prefill_exact(prev)
 
 
+@pytest.mark.parametrize("M,H,HK", [(672, 48, 16), (673, 48, 16), (70, 5, 2), (70, 3, 5)])
+def test_gdn_chunked_prep_split(q27, dev, M, H, HK):
+    """One preparing workgroup per value head up to 1024 of them (672 tokens of 48 heads: 1008), per key head beyond
+    (673 tokens: 1056); a last set of value heads that covers only some key heads; more key heads than value heads."""
+    say(f"gdn chunked prep split M={M} H={H} HK={HK}")
+    x, stride, g, beta, planes = cd.gdn_inputs(cd.rng(900 + M + H), M, H, HK)
+    got_o, got_p = _run(q27, dev, x, stride, g, beta, planes, 0, H, HK, M)
+    want_o, want_s = _f64_recurrence(x, stride, g, beta, planes, 0, H, HK, M)
+    n = H * 128 * 128
+    _close(got_o, want_o, f"o vs float64 M={M} H={H} HK={HK}", RTOL_F64)
+    _close(got_p[n:2 * n], want_s, f"state vs float64 M={M} H={H} HK={HK}", RTOL_F64)
+
+
 @pytest.mark.parametrize("stride", [1 << 24, (1 << 24) + 4])
 def test_gdn_chunked_wide_rows(q27, dev, stride):
     """Rows 2^24 floats apart (the last stride whose chunk the 32-bit offsets reach: the bits of compact rows) and
