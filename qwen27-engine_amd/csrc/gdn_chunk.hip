@@ -301,7 +301,8 @@ __global__ void __launch_bounds__(512) gdn_chunk_kernel(const float* __restrict_
   float4 pk[2], pq[2];
   float pv[2], pt[2], pg = 0.0f, pb = 0.0f;
   // Chunk ch's rows into registers, through buffer descriptors of the chunk's rows: reads past its last token return
-  // zeros, so no load is conditional and the compiler's waits count them exactly.
+  // zeros, so no load is conditional and the compiler's waits count them exactly. The whole row offset is in the vector
+  // offset: the bounds check is only specified for that one, not for the scalar offset.
   auto rows_of = [&](const float* p, int c0, int n, int ld, int width) {
     return __builtin_amdgcn_make_buffer_rsrc((void*)(p + (n > 0 ? (size_t)c0 * ld : 0)), 0, n > 0 ? ((n - 1) * ld + width) * 4 : 0,
                                              0x00027000);
@@ -319,12 +320,13 @@ __global__ void __launch_bounds__(512) gdn_chunk_kernel(const float* __restrict_
     const int pl = full ? (st_t * H * 128 + st_c) * 4 : (st_c * 128 + st_t) * 4, ps = full ? 16 * H * 128 * 4 : 16 * 4;
 #pragma unroll
     for (int u = 0; u < 2; u++) {
-      const v4f a = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(fk, (st_t * stride + st_e4) * 4, 16 * u * stride * 4, 0));
-      const v4f b = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(fq, (st_t * stride + st_e4) * 4, 16 * u * stride * 4, 0));
+      const int row = (st_t + 16 * u) * stride;
+      const v4f a = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(fk, (row + st_e4) * 4, 0, 0));
+      const v4f b = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(fq, (row + st_e4) * 4, 0, 0));
       pk[u] = make_float4(a[0], a[1], a[2], a[3]);
       pq[u] = make_float4(b[0], b[1], b[2], b[3]);
-      const uint32_t c = __builtin_amdgcn_raw_buffer_load_b32(fv, (st_t * stride + st_c) * 4, 16 * u * stride * 4, 0);
-      const uint32_t d = __builtin_amdgcn_raw_buffer_load_b32(fp, pl, u * ps, 0);
+      const uint32_t c = __builtin_amdgcn_raw_buffer_load_b32(fv, (row + st_c) * 4, 0, 0);
+      const uint32_t d = __builtin_amdgcn_raw_buffer_load_b32(fp, pl + u * ps, 0, 0);
       pv[u] = __builtin_bit_cast(float, c);
       pt[u] = __builtin_bit_cast(float, d);
     }

@@ -182,6 +182,29 @@ def test_gdn_chunked_prep_split(q27, dev, M, H, HK):
     _close(got_p[n:2 * n], want_s, f"state vs float64 M={M} H={H} HK={HK}", RTOL_F64)
 
 
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 31])
+def test_gdn_chunked_ragged_rows_inside_a_larger_batch(q27, dev, n):
+    """Every row behind the last token is NaN (x, g, beta): a last chunk of n tokens gives the bits of the compact batch,
+    and the rows of o behind it are not written."""
+    import torch
+
+    H, HK, M, pad = 6, 2, 32 + n, 32
+    say(f"gdn chunked ragged n={n}")
+    x, W, g, beta, planes = cd.gdn_inputs(cd.rng(950 + n), M, H, HK)
+    want_o, want_p = _run(q27, dev, x, W, g, beta, planes, 0, H, HK, M)
+    dx, dg, db = (torch.cat([torch.from_numpy(a).to(dev), torch.full((pad * w,), float("nan"), device=dev)])
+                  for a, w in ((x, W), (g, H), (beta, H)))
+    dp = torch.from_numpy(planes).to(dev)
+    pin = torch.zeros(1, dtype=torch.int32, device=dev)
+    o = torch.full(((M + pad) * H * 128,), -7.0, device=dev)
+    q27.ops.gdn_step_chunked(dx, dx[HK * 128:], dx[2 * HK * 128:], W, dg, db, dp, pin, o, H, HK, M, float(SCALE))
+    torch.cuda.synchronize()
+    got = o.cpu().numpy()
+    assert np.array_equal(got[: M * H * 128].view(np.uint32), want_o.view(np.uint32))
+    assert np.array_equal(dp.cpu().numpy().view(np.uint32), want_p.view(np.uint32))
+    assert np.all(got[M * H * 128:] == -7.0)
+
+
 @pytest.mark.parametrize("stride", [1 << 24, (1 << 24) + 4])
 def test_gdn_chunked_wide_rows(q27, dev, stride):
     """Rows 2^24 floats apart (the last stride whose chunk the 32-bit offsets reach: the bits of compact rows) and
