@@ -262,6 +262,10 @@ gdn_chunk_prep_kernel(const float* __restrict__ q, const float* __restrict__ k, 
 }
 
 // ---------------------------------------------------------------- the recurrence over the chunks
+// WIDE: 64-bit row offsets and a condition per row instead of buffer descriptors, whose 32-bit offsets inside a chunk's
+// 32 rows end at rows of 2^24 floats (64 MB): 256 tokens 2^24 + 4 floats apart 41.9 us (the sequential kernel 66.9).
+constexpr bool wide_rows(int stride, int H) { return stride > (1 << 24) || H > (1 << 17); }
+template <bool WIDE>
 __global__ void __launch_bounds__(512) gdn_chunk_kernel(const float* __restrict__ q, const float* __restrict__ k,
                                                         const float* __restrict__ v, int stride,
                                                         const float* __restrict__ g, const float* __restrict__ beta,
@@ -309,6 +313,20 @@ __global__ void __launch_bounds__(512) gdn_chunk_kernel(const float* __restrict_
   };
   auto fetch = [&](int ch) {
     const int c0 = ch * kC, n = min(kC, T - c0);
+    if constexpr (WIDE) {
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        const int t = st_t + 16 * u;
+        const size_t row = (size_t)(c0 + t) * stride;
+        pk[u] = t < n ? ld4(k + row + kh * 128 + st_e4) : make_float4(0.f, 0.f, 0.f, 0.f);
+        pq[u] = t < n ? ld4(q + row + kh * 128 + st_e4) : make_float4(0.f, 0.f, 0.f, 0.f);
+        pv[u] = t < n ? v[row + h * 128 + cg * kNC + st_c] : 0.0f;
+        if (n == kC) pt[u] = o[((size_t)(c0 + t) * H + h) * 128 + cg * kNC + st_c];
+        else if (n > 0) pt[u] = planes[(size_t)pout * plane_sz + ((size_t)h * 128 + cg * kNC + st_c) * 128 + t];
+        else pt[u] = 0.0f;
+      }
+      return;
+    }
     const auto fk = rows_of(k + kh * 128, c0, n, stride, 128), fq = rows_of(q + kh * 128, c0, n, stride, 128);
     const auto fv = rows_of(v + h * 128 + cg * kNC, c0, n, stride, kNC);
     // P: parked in o's rows for a full chunk, else in the output plane (column st_c, key t)
@@ -333,6 +351,11 @@ __global__ void __launch_bounds__(512) gdn_chunk_kernel(const float* __restrict_
   };
   auto fetch_g = [&](int ch) {  // wave 1: g and beta, token l on lane l
     const int c0 = ch * kC, n = min(kC, T - c0);
+    if constexpr (WIDE) {
+      pg = l < n ? g[(size_t)(c0 + l) * H + h] : 0.0f;
+      pb = l < n ? beta[(size_t)(c0 + l) * H + h] : 0.0f;
+      return;
+    }
     const auto fg = rows_of(g + h, c0, n, H, 1), fb = rows_of(beta + h, c0, n, H, 1);
     const uint32_t a = __builtin_amdgcn_raw_buffer_load_b32(fg, l * H * 4, 0, 0);
     const uint32_t b = __builtin_amdgcn_raw_buffer_load_b32(fb, l * H * 4, 0, 0);
@@ -485,12 +508,20 @@ __global__ void __launch_bounds__(512) gdn_chunk_kernel(const float* __restrict_
 #pragma unroll
         for (int m = 4; m < 8; m++) oz = mfma4(mo[m], dl[m], oz);
       }
-      const auto fo = rows_of(o + h * 128, c0, n, H * 128, 128);  // (stores past the last token are dropped)
+      if constexpr (WIDE) {
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const float x = oz[i] * scale;
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), fo,
-                                              ((16 * ot + 4 * kq + i) * H * 128 + cg * kNC + cb * 16 + r) * 4, 0, 0);
+        for (int i = 0; i < 4; i++) {
+          const int t = 16 * ot + 4 * kq + i;
+          if (t < n) o[((size_t)(c0 + t) * H + h) * 128 + col] = oz[i] * scale;
+        }
+      } else {
+        const auto fo = rows_of(o + h * 128, c0, n, H * 128, 128);  // (stores past the last token are dropped)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const float x = oz[i] * scale;
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), fo,
+                                                ((16 * ot + 4 * kq + i) * H * 128 + cg * kNC + cb * 16 + r) * 4, 0, 0);
+        }
       }
     }
     if (!early) {
@@ -533,14 +564,12 @@ extern "C" int q27h_gdn_step_chunked(const float* q, const float* k, const float
   if (gdn_chunk_o_overlaps(q, k, v, stride, g, beta, planes, o, H, HK, T))
     return fail(Q27H_ERR_ARG, "gdn_step_chunked: o overlaps q / k / v rows, g, beta or the state planes");
   const hipStream_t st = stream_of(s);
-  if (!gdn_chunk_fits(stride, H))  // the sequential kernel's 64-bit offsets
-    return gdn_prefill_sequential(q, k, v, stride, g, beta, planes, in_plane, o, H, HK, T, scale, st);
   const int keys = min(H, HK), chunks = (T + kC - 1) / kC, heads = (H + HK - 1) / HK;
   const int split = (long)keys * chunks * heads <= kPrepResident ? heads : 1;
   hipLaunchKernelGGL(gdn_chunk_prep_kernel, dim3(keys, chunks, split), dim3(256), 0, st, q, k, stride, g, beta,
                      planes, in_plane, o, H, HK, T);
   if (int e = check_launch("gdn_step_chunked")) return e;
-  hipLaunchKernelGGL(gdn_chunk_kernel, dim3(H, 128 / kNC), dim3(512), 0, st, q, k, v, stride, g, beta, planes, in_plane,
-                     o, H, HK, T, scale);
+  hipLaunchKernelGGL(wide_rows(stride, H) ? gdn_chunk_kernel<true> : gdn_chunk_kernel<false>, dim3(H, 128 / kNC), dim3(512),
+                     0, st, q, k, v, stride, g, beta, planes, in_plane, o, H, HK, T, scale);
   return check_launch("gdn_step_chunked");
 }

@@ -27,10 +27,5 @@ bool gdn_prefill_exact_mode();
 // gdn_chunk.hip: whether o shares memory with an input of the chunked delta-rule prefill (which it may not).
 bool gdn_chunk_o_overlaps(const float* q, const float* k, const float* v, int stride, const float* g, const float* beta,
                           const float* planes, const float* o, int H, int HK, int T);
-// Row strides and head counts the chunked kernel's 32-bit offsets inside a chunk's 32 rows reach (a row of 64 MB).
-inline bool gdn_chunk_fits(int stride, int H) { return stride <= (1 << 24) && H <= (1 << 17); }
-// gdn_rec.hip: the sequential prefill launch (arguments already checked).
-int gdn_prefill_sequential(const float* q, const float* k, const float* v, int stride, const float* g, const float* beta,
-                           float* planes, const int* in_plane, float* o, int H, int HK, int T, float scale, hipStream_t s);
 
 }  // namespace q27h

@@ -207,22 +207,14 @@ def test_gdn_chunked_ragged_rows_inside_a_larger_batch(q27, dev, n):
 
 @pytest.mark.parametrize("stride", [1 << 24, (1 << 24) + 4])
 def test_gdn_chunked_wide_rows(q27, dev, stride):
-    """Rows 2^24 floats apart (the last stride whose chunk the 32-bit offsets reach: the bits of compact rows) and
-    farther (the sequential kernel: its bits). 65 rows: a full chunk, a second one and a ragged one."""
+    """Rows 2^24 floats apart (the last stride whose chunk 32-bit offsets reach) and farther (64-bit offsets): the bits of
+    compact rows. 65 rows: a full chunk, a second one and a ragged one."""
     import torch
 
     H, HK, M = 2, 1, 65
     say(f"gdn chunked stride={stride}")
     x, W, g, beta, planes = cd.gdn_inputs(cd.rng(800), M, H, HK)
-    prev = q27.ops.gdn_prefill_exact(False)
-    try:
-        if stride <= 1 << 24:
-            want_o, want_p = _run(q27, dev, x, W, g, beta, planes, 0, H, HK, M)
-        else:
-            q27.ops.gdn_prefill_exact(True)
-            want_o, want_p = _run_step(q27, dev, x, W, g, beta, planes, 0, H, HK, M)
-    finally:
-        q27.ops.gdn_prefill_exact(prev)
+    want_o, want_p = _run(q27, dev, x, W, g, beta, planes, 0, H, HK, M)
     dx = torch.empty((M - 1) * stride + W, device=dev)
     dx.as_strided((M, W), (stride, 1)).copy_(torch.from_numpy(x).to(dev).view(M, W))
     dp = torch.from_numpy(planes).to(dev)
