@@ -1040,13 +1040,18 @@ constexpr bool folds(int type, int nc) { return (nc == 2 || nc == 3) && (type ==
 // 15.8 -> 13.4, IQ1_M 17.1 -> 15.0).
 // Three columns in one launch (two launches before: every weight read and decoded twice), us, 17408 x 5120 / 5120 x 17408:
 // Q4_K 22.1 -> 14.4 / 23.4 -> 16.1, Q6_K 28.9 -> 18.3 / 30.5 -> 24.7, IQ2_XS 23.9 -> 17.1 / 22.9 -> 18.5, IQ4_XS 24.7 ->
-// 15.9 / 25.7 -> 17.8, IQ3_S 26.6 -> 15.6, IQ1_M 27.5 -> 21.6; smaller matrices (1024 x 5120, 2048 x 1024) 1.4-1.7 times as
+// 15.9 / 25.7 -> 17.8, IQ3_S 26.6 -> 15.6, IQ1_M 27.6 -> 20.3; smaller matrices (1024 x 5120, 2048 x 1024) 1.4-1.7 times as
 // fast. 6 waves per SIMD (80 VGPRs) instead of 4 also let two workgroups of nine waves (K = 17408) share a CU
 // (us, 17408 x 5120 / 5120 x 17408, 4 -> 6: Q4_K 16.3 / 22.7 -> 14.4 / 16.1, IQ2_XS 20.1 / 25.6 -> 17.1 / 18.5, IQ4_XS
 // 18.3 / 22.3 -> 15.9 / 17.8); Q6_K spills at 6 (27.3 / 28.8, at 5 18.3 / 24.7), IQ3_XXS and IQ3_S run slower (16.4 and
-// 16.5, at 5 15.5 and 15.6).
+// 16.5, at 5 15.5 and 15.6). IQ1_M needs 98 VGPRs and spills at 6 (68 bytes of scratch per lane) and at 5 (8 bytes): 4
+// (17408 x 5120 / 5120 x 8192 / 1024 x 5120: 21.3 / 12.2 / 6.3 at 6, 20.3 / 10.8 / 6.3 at 4; f32 activations 60.9 / 27.8 /
+// 12.7 -> 58.9 / 26.0 / 12.4).
+// With f32 activations 58 KB of LDS allow two workgroups per CU whatever the registers, and the fewer registers still
+// gain (17408 x 5120 / 1024 x 5120, uncapped -> capped): IQ2_S of four columns 72.6 / 14.7 -> 70.0 / 14.2, although one
+// register spills (8 bytes of scratch per lane); two columns IQ3_S 35.2 / 9.3 -> 32.6 / 8.8, IQ1_M 45.2 / 9.3 -> 42.2 / 8.9.
 constexpr int one_waves_per_simd(int type, int nc) {
-  if (nc == 3) return type == kQ6K || type == kIQ3XXS || type == kIQ3S ? 5 : 6;
+  if (nc == 3) return type == kIQ1M ? 4 : type == kQ6K || type == kIQ3XXS || type == kIQ3S ? 5 : 6;
   if (nc == 2) return folds(type, 2) ? 6 : 4;
   if (nc == 4) return type == kIQ2S ? 5 : 4;
   return 4;
