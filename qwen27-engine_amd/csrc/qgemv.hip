@@ -14,12 +14,10 @@
 // The same summation order is restated by the CPU checker, so results are bit-identical to it.
 #include "q27h_device.h"
 #include "q27h_internal.h"
+#include "qgemv_route.h"
 
 namespace q27h {
 namespace {
-
-constexpr int kQ2K = 10, kQ4K = 12, kQ6K = 14, kIQ2XXS = 16, kIQ2XS = 17, kIQ3XXS = 18, kIQ3S = 21, kIQ2S = 22,
-              kIQ4XS = 23, kIQ1M = 29;
 
 __device__ const __align__(16) uint32_t kIQ3SGrid[512] = {
 #include "iq3s_grid.inc"
@@ -840,24 +838,10 @@ __device__ __forceinline__ void reduce_level(float (&a)[V], int lane) {
     a[0] += xchg<O>(a[0]);
   }
 }
-// Waves per tile, a function of the type, K and the column count only (part of the summation order). One column, and
-// two for all types but IQ3_XXS / IQ3_S / IQ1_M: one block of each tile per lane, ceil(K / 2048) waves, up to K = 32768
-// (16 waves); each wave adds a butterfly, which is cheap for few columns. Otherwise, and for K > 32768: at most 4 waves,
-// lanes taking several blocks. Measured (us, 5120 x 17408, 4 -> 9 waves): T = 1 Q4_K 13.1 -> 10.9, IQ3_S 18.0 -> 12.5,
-// IQ2_XXS 14.7 -> 9.7; T = 2 Q4_K 14.7 -> 13.5, IQ2_S 19.3 -> 14.7, but IQ3_S 15.8 -> 20.1, IQ1_M 18.1 -> 21.5; T = 4
-// Q4_K 18.7 -> 25.4.
-constexpr int kMaxW = 16;
-constexpr int waves_per_tile(int type, int K, int ncols) {
-  const int w = (K / 256 + 7) / 8;
-  const bool wide = ncols == 1 || (ncols == 2 && type != kIQ3XXS && type != kIQ3S && type != kIQ1M);
-  const int cap = wide ? kMaxW : 4;
-  return w < 1 ? 1 : w > kMaxW ? 4 : w > cap ? cap : w;
-}
 
 // FUSED: the activations arrive as f32 (xf, [NC][K]); every workgroup first quantizes them to q8_1 in LDS with the
 // code of quantize_q8_1 (q8_1_store_n: amax, d = amax / 127, q = roundf(y / d), scale fp16(d)), then reads them from
 // there. The results are those of quantize_q8_1 followed by the unfused GEMV, bit for bit.
-constexpr int kFusedMaxX = 40960;  // NC * K values a fused launch may quantize per workgroup (40 KB of int8 in LDS)
 // FOLD: every wave of the workgroup takes one block per lane as in ONE, but the sums are those of W waves whose lanes
 // take several blocks: before the butterfly the waves W, W + 1, ... hand their lanes' sums over in LDS, and wave w adds
 // those of w + W, w + 2 W, ... in order (a lane without a block has +0). Of three columns the third is ordered by one
@@ -1019,13 +1003,6 @@ __device__ __forceinline__ void qgemv_body(Mat m, const int8_t* __restrict__ xq,
   }
 }
 
-// IQ3_XXS / IQ3_S / IQ1_M, two or three columns, 8192 < K <= 32768: 4 waves' sums formed by one block per lane. Three
-// columns ran as launches of two and one, two on the prefetching kernel. Measured (us, 5120 x 17408 / 5120 x 10240 / 1024 x
-// 20480): T = 3 IQ3_S 27.3 / 19.6 / 15.8 -> 19.2 / 12.2 / 9.6, IQ3_XXS 26.4 / 18.7 / 16.2 -> 19.0 / 12.0 / 9.5, IQ1_M 28.8 /
-// 20.7 / 17.4 -> 28.8 / 14.4 / 11.5; T = 2 IQ3_S 17.4 / 12.0 / 9.6 -> 17.5 / 10.8 / 8.4, IQ3_XXS 16.9 / 11.6 / 10.3 -> 16.4 /
-// 10.2 / 8.1, IQ1_M 18.8 / 13.3 / 11.3 -> 16.9 / 11.1 / 8.7. Four columns ran slower (5120 x 17408 Q4_K 18.6 -> 24-26, IQ3_S
-// 20.9 -> 27.7: 9 waves of 96 VGPRs and 40 KB per workgroup, 640 workgroups are 1.25 rounds of the CUs).
-constexpr bool folds(int type, int nc) { return (nc == 2 || nc == 3) && (type == kIQ3XXS || type == kIQ3S || type == kIQ1M); }
 // Kernel for K <= 2048 W (every lane takes at most one block of its tile): no prefetch registers, and the compiler is
 // held to 128 VGPRs (4 waves per SIMD) for four columns. Measured against the prefetching kernel (us, 17408 x 5120,
 // T = 1 / T = 4): Q4_K 10.9 -> 9.8 / 17.3 -> 17.9, Q6_K 14.7 -> 13.1 / 20.0 -> 19.3, IQ3_S 13.2 -> 11.4 / 20.3 -> 19.3,
@@ -1068,9 +1045,6 @@ qgemv_one_kernel(Mat m, const int8_t* __restrict__ xq, const float* __restrict__
   qgemv_body<TYPE, NC, true, true, FUSED>(m, xq, xd, y, K, W, xf);
 }
 
-// Three columns: the order of the sums is that of two columns, then that of one. Whether both take the same waves (all but
-// IQ3_XXS / IQ3_S / IQ1_M at 8192 < K <= 32768, which need the folding kernel).
-constexpr bool three_alike(int type, int K) { return waves_per_tile(type, K, 2) == waves_per_tile(type, K, 1); }
 template <int TYPE, int NC>
 __global__ void __launch_bounds__(64 * kMaxW) __attribute__((amdgpu_waves_per_eu(NC == 3 ? 5 : 6)))
 qgemv_fold_kernel(Mat m, const int8_t* __restrict__ xq, const float* __restrict__ xd, float* __restrict__ y, int K, int W) {
@@ -1089,8 +1063,8 @@ void launch_gemv(const Mat& m, const int8_t* xq, const float* xd, float* y, int 
   // the prefetching kernel takes at most 4 waves (lanes with several blocks); W > 4 means one block per lane
   const bool one = m.nb <= 8 * W && (W > 4 || !((TYPE == kQ2K || TYPE == kQ4K) && NC == 4));
   if constexpr (!FUSED && folds(TYPE, NC)) {
-    const int g = (m.nb + 7) / 8;
-    if (g > W && g <= kMaxW) {
+    if (fold_pays(TYPE, K, NC, m.ntiles)) {
+      const int g = (m.nb + 7) / 8;
       hipLaunchKernelGGL((qgemv_fold_kernel<TYPE, NC>), dim3(grid), dim3(64 * g), (g - W) * 16 * 256, s, m, xq, xd, y, K, W);
       return;
     }
@@ -1108,8 +1082,14 @@ void launch_nc(const Mat& m, const int8_t* xq, const float* xd, float* y, int K,
                const float* xf = nullptr) {
   if (nc == 1) launch_gemv<TYPE, 1, FUSED>(m, xq, xd, y, K, s, xf);
   else if (nc == 2) launch_gemv<TYPE, 2, FUSED>(m, xq, xd, y, K, s, xf);
-  else if (nc == 3) launch_gemv<TYPE, 3, FUSED>(m, xq, xd, y, K, s, xf);
-  else launch_gemv<TYPE, 4, FUSED>(m, xq, xd, y, K, s, xf);
+  else if (nc == 3) {
+    if (three_in_one(TYPE, K, m.ntiles, FUSED)) return launch_gemv<TYPE, 3, FUSED>(m, xq, xd, y, K, s, xf);
+    const size_t k2 = (size_t)2 * K;
+    launch_gemv<TYPE, 2, FUSED>(m, xq, xd, y, K, s, xf);
+    float* y2 = y + (size_t)2 * m.N;
+    if constexpr (FUSED) launch_gemv<TYPE, 1, true>(m, xq, xd, y2, K, s, xf + k2);
+    else launch_gemv<TYPE, 1>(m, xq + k2, xd + k2 / 32, y2, K, s);
+  } else launch_gemv<TYPE, 4, FUSED>(m, xq, xd, y, K, s, xf);
 }
 
 }  // namespace
@@ -1197,25 +1177,17 @@ extern "C" int q27h_qgemv_f32(int type, int N, int K, const void* buf, const flo
   const uint8_t* b = (const uint8_t*)buf;
   const Mat m{{b + off[0], b + off[1], b + off[2], b + off[3]}, b + off[4], N, K / 256, N / 8};
   const hipStream_t st = stream_of(s);
-  auto run = [&](const float* xx, float* yy, int nc) {
-    switch (type) {
-      case kQ2K: launch_nc<kQ2K, true>(m, nullptr, nullptr, yy, K, nc, st, xx); break;
-      case kQ4K: launch_nc<kQ4K, true>(m, nullptr, nullptr, yy, K, nc, st, xx); break;
-      case kQ6K: launch_nc<kQ6K, true>(m, nullptr, nullptr, yy, K, nc, st, xx); break;
-      case kIQ2XXS: launch_nc<kIQ2XXS, true>(m, nullptr, nullptr, yy, K, nc, st, xx); break;
-      case kIQ2XS: launch_nc<kIQ2XS, true>(m, nullptr, nullptr, yy, K, nc, st, xx); break;
-      case kIQ3XXS: launch_nc<kIQ3XXS, true>(m, nullptr, nullptr, yy, K, nc, st, xx); break;
-      case kIQ3S: launch_nc<kIQ3S, true>(m, nullptr, nullptr, yy, K, nc, st, xx); break;
-      case kIQ2S: launch_nc<kIQ2S, true>(m, nullptr, nullptr, yy, K, nc, st, xx); break;
-      case kIQ1M: launch_nc<kIQ1M, true>(m, nullptr, nullptr, yy, K, nc, st, xx); break;
-      default: launch_nc<kIQ4XS, true>(m, nullptr, nullptr, yy, K, nc, st, xx); break;
-    }
-  };
-  if (ncols == 3 && !(three_alike(type, K) && (long)K * 3 <= kFusedMaxX)) {
-    run(x, y, 2);
-    run(x + (size_t)2 * K, y + (size_t)2 * N, 1);
-  } else {
-    run(x, y, ncols);
+  switch (type) {
+    case kQ2K: launch_nc<kQ2K, true>(m, nullptr, nullptr, y, K, ncols, st, x); break;
+    case kQ4K: launch_nc<kQ4K, true>(m, nullptr, nullptr, y, K, ncols, st, x); break;
+    case kQ6K: launch_nc<kQ6K, true>(m, nullptr, nullptr, y, K, ncols, st, x); break;
+    case kIQ2XXS: launch_nc<kIQ2XXS, true>(m, nullptr, nullptr, y, K, ncols, st, x); break;
+    case kIQ2XS: launch_nc<kIQ2XS, true>(m, nullptr, nullptr, y, K, ncols, st, x); break;
+    case kIQ3XXS: launch_nc<kIQ3XXS, true>(m, nullptr, nullptr, y, K, ncols, st, x); break;
+    case kIQ3S: launch_nc<kIQ3S, true>(m, nullptr, nullptr, y, K, ncols, st, x); break;
+    case kIQ2S: launch_nc<kIQ2S, true>(m, nullptr, nullptr, y, K, ncols, st, x); break;
+    case kIQ1M: launch_nc<kIQ1M, true>(m, nullptr, nullptr, y, K, ncols, st, x); break;
+    default: launch_nc<kIQ4XS, true>(m, nullptr, nullptr, y, K, ncols, st, x); break;
   }
   return check_launch("qgemv_f32");
 }

@@ -97,6 +97,29 @@ def test_qgemv_three_columns(q27, oracle, dev, type_, N, K, f32):
     assert_bits_equal(got, np.asarray(want).reshape(3, N), f"qgemv three columns type {type_} {N}x{K}")
 
 
+@pytest.mark.parametrize("type_,N,K,ncols", [
+    (21, 6144, 17408, 2), (21, 6152, 17408, 2), (18, 6152, 24576, 2), (21, 2048, 24832, 2), (21, 2056, 24832, 2),
+    (18, 4104, 32768, 2), (29, 4104, 24832, 2), (29, 10248, 17408, 3), (29, 16392, 18688, 3), (29, 16384, 18688, 3),
+    (18, 24, 8448, 2), (21, 24, 8448, 2), (29, 24, 8448, 2)])
+def test_qgemv_folding_routes(q27, oracle, dev, type_, N, K, ncols):
+    """The folding kernel and the route beside it, on both sides of the lines between them (matrices of 40 distinct rows),
+    and the first K that folds (5 waves)."""
+    import torch
+
+    say(f"qgemv folding routes type {type_} {N}x{K} ncols={ncols}")
+    r = cd.rng(520 + type_ + N + K)
+    rows = min(N, 40)
+    raw = cd.random_weights(r, type_, rows, K)
+    xq, xd = cd.q8_activations(oracle, r, ncols, K)
+    want = np.asarray(oracle.qgemv(type_, raw, rows, K, xq, xd, ncols)).reshape(ncols, rows)
+    draw = torch.from_numpy(np.ascontiguousarray(raw)).to(dev).view(torch.uint8).view(rows, -1)
+    m = q27.ops.qmat_upload(draw.repeat(-(-N // rows), 1)[:N].contiguous().view(-1), type_, N, K)
+    y = torch.full((ncols * N,), float("nan"), device=dev)
+    q27.ops.qgemv(m, torch.from_numpy(xq).to(dev), torch.from_numpy(xd).to(dev), y, ncols)
+    got = y.cpu().numpy().reshape(ncols, N)
+    assert_bits_equal(got, np.tile(want, (1, -(-N // rows)))[:, :N], f"qgemv type {type_} {N}x{K} ncols {ncols}")
+
+
 def test_qgemv_small_and_edge_shapes(q27, oracle, dev):
     """One tile, one block per row, and partial 8-block groups; zero activations and wide scale ranges."""
     for type_ in TYPES:
