@@ -373,7 +373,6 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // 14.4 / 13.8, IQ4_XS 15.9 / 15.0, Q2_K 11.1 / 10.6; 17408 x 5120 Q6_K 14.6 / 15.2, Q4_K 11.0 / 11.4, IQ4_XS 12.1 /
 // 12.7. rocprofv3 FETCH_SIZE shows why: with nontemporal pieces a 5120 x 17408 Q6_K launch fetches 98 MB for its
 // 73 MB matrix, with ordinary loads 75-77 MB.
-constexpr int kNtPiecesMaxK = 8192;
 #ifndef Q27H_QG_NT_SMALL
 #define Q27H_QG_NT_SMALL 1
 #endif
@@ -1060,8 +1059,6 @@ template <int TYPE, int NC, bool FUSED = false>
 void launch_gemv(const Mat& m, const int8_t* xq, const float* xd, float* y, int K, hipStream_t s, const float* xf = nullptr) {
   const int W = waves_per_tile(TYPE, K, NC == 3 ? 2 : NC);
   const int grid = m.ntiles;
-  // the prefetching kernel takes at most 4 waves (lanes with several blocks); W > 4 means one block per lane
-  const bool one = m.nb <= 8 * W && (W > 4 || !((TYPE == kQ2K || TYPE == kQ4K) && NC == 4));
   if constexpr (!FUSED && folds(TYPE, NC)) {
     if (fold_pays(TYPE, K, NC, m.ntiles)) {
       const int g = (m.nb + 7) / 8;
@@ -1069,12 +1066,16 @@ void launch_gemv(const Mat& m, const int8_t* xq, const float* xd, float* y, int 
       return;
     }
   }
-  if (one)
-    hipLaunchKernelGGL((qgemv_one_kernel<TYPE, NC, FUSED>), dim3(grid), dim3(64 * W), 0, s, m, xq, xd, y, K, W, xf);
-  else if (K <= kNtPiecesMaxK)
-    hipLaunchKernelGGL((qgemv_kernel<TYPE, NC, true, FUSED>), dim3(grid), dim3(64 * W), 0, s, m, xq, xd, y, K, W, xf);
-  else
-    hipLaunchKernelGGL((qgemv_kernel<TYPE, NC, false, FUSED>), dim3(grid), dim3(64 * W), 0, s, m, xq, xd, y, K, W, xf);
+  if (one_block(TYPE, K, NC)) {
+    if constexpr (one_block_reached(TYPE, NC))
+      hipLaunchKernelGGL((qgemv_one_kernel<TYPE, NC, FUSED>), dim3(grid), dim3(64 * W), 0, s, m, xq, xd, y, K, W, xf);
+  } else if (K <= kNtPiecesMaxK) {
+    if constexpr (prefetch_reached(TYPE, NC, FUSED, true))
+      hipLaunchKernelGGL((qgemv_kernel<TYPE, NC, true, FUSED>), dim3(grid), dim3(64 * W), 0, s, m, xq, xd, y, K, W, xf);
+  } else {
+    if constexpr (prefetch_reached(TYPE, NC, FUSED, false))
+      hipLaunchKernelGGL((qgemv_kernel<TYPE, NC, false, FUSED>), dim3(grid), dim3(64 * W), 0, s, m, xq, xd, y, K, W, xf);
+  }
 }
 
 template <int TYPE, bool FUSED = false>

@@ -52,12 +52,29 @@ constexpr bool fold_pays(int type, int K, int nc, int tiles) {
   return tiles <= (type == kIQ3S ? 256 : 512);
 }
 
+// One block per lane, without prefetch registers (up to 4 waves Q2_K and Q4_K of four columns keep the prefetching kernel:
+// 17408 x 5120 17.2 / 17.3 us against 18.8 / 17.9).
+constexpr bool one_block(int type, int K, int nc) {
+  const int w = waves_per_tile(type, K, nc == 3 ? 2 : nc);
+  return K / 256 <= 8 * w && (w > 4 || !((type == kQ2K || type == kQ4K) && nc == 4));
+}
+
 // Three columns: the order of the sums is that of two columns, then that of one. One launch where both take the same waves
 // (all but IQ3_XXS / IQ3_S / IQ1_M at 8192 < K <= 32768), or with the folding kernel; over f32 activations where they fit.
+constexpr bool three_alike(int type, int K) { return waves_per_tile(type, K, 2) == waves_per_tile(type, K, 1); }
 constexpr bool three_in_one(int type, int K, int tiles, bool fused) {
-  const bool alike = waves_per_tile(type, K, 2) == waves_per_tile(type, K, 1);
-  if (fused) return alike && (long)K * 3 <= kFusedMaxX;
-  return alike || fold_pays(type, K, 3, tiles);
+  if (fused) return three_alike(type, K) && (long)K * 3 <= kFusedMaxX;
+  return three_alike(type, K) || fold_pays(type, K, 3, tiles);
+}
+
+// Whether some K takes a kernel at all; the others are not built. The prefetching kernel reads a tile's wide pieces with
+// nontemporal loads up to kNtPiecesMaxK and is the only one beyond K = 32768.
+constexpr int kNtPiecesMaxK = 8192;
+constexpr bool one_block_reached(int type, int nc) { return one_block(type, 256, nc); }
+constexpr bool prefetch_reached(int type, int nc, bool fused, bool nt) {
+  for (int K = 256; K <= (fused ? kFusedMaxX / nc : 33024); K += 256)
+    if (!one_block(type, K, nc) && (K <= kNtPiecesMaxK) == nt && (nc != 3 || three_alike(type, K))) return true;
+  return false;
 }
 
 }  // namespace q27h

@@ -3,15 +3,19 @@ take the folding kernel, and which three-column calls are one launch. Both route
 depends on the lines checked here; each case is a call just inside and just outside of one."""
 import ctypes
 import os
+import re
 import subprocess
 
 import pytest
+
+import codeobj
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "qwen27-engine_amd", "csrc")
 SRC = """
 #include "qgemv_route.h"
 using namespace q27h;
 extern "C" int fold(int type, int K, int nc, int tiles) { return fold_pays(type, K, nc, tiles); }
+extern "C" int one(int type, int K, int nc) { return one_block(type, K, nc); }
 extern "C" int three(int type, int K, int tiles, int fused) { return three_in_one(type, K, tiles, fused != 0); }
 """
 IQ3_XXS, IQ3_S, IQ1_M = 18, 21, 29
@@ -58,3 +62,25 @@ def test_three_columns_in_one_launch(route):
             for tiles in (1, 640, 5000):
                 assert route.three(type_, K, tiles, 0) == (not differ or route.fold(type_, K, 3, tiles))
                 assert route.three(type_, K, tiles, 1) == (not differ and 3 * K <= 40960)
+
+
+def test_built_kernels_are_those_some_call_takes(route):
+    """Every instantiation that a call of some K and number of tiles takes is in the library, and no other."""
+    want = set()
+    for type_ in TYPES:
+        for nc in (1, 2, 3, 4):
+            for fused in (0, 1):
+                for K in range(256, 40961, 256):
+                    if fused and (2 if nc == 3 else nc) * K > 40960:
+                        continue
+                    for tiles in (1, 1 << 20):
+                        cols = [nc] if nc != 3 or route.three(type_, K, tiles, fused) else [2, 1]
+                        for c in cols:
+                            if not fused and route.fold(type_, K, c, tiles):
+                                want.add(f"qgemv_fold_kernelILi{type_}ELi{c}EE")
+                            elif route.one(type_, K, c):
+                                want.add(f"qgemv_one_kernelILi{type_}ELi{c}ELb{fused}EE")
+                            else:
+                                want.add(f"qgemv_kernelILi{type_}ELi{c}ELb{int(K <= 8192)}ELb{fused}EE")
+    built = {re.search(r"qgemv\w*?_kernelI\w*?EE", n).group(0) for n in codeobj.kernels() if "qgemv" in n}
+    assert built == want, (sorted(want - built), sorted(built - want))
