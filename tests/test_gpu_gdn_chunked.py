@@ -182,6 +182,19 @@ def test_gdn_chunked_prep_split(q27, dev, M, H, HK):
     _close(got_p[n:2 * n], want_s, f"state vs float64 M={M} H={H} HK={HK}", RTOL_F64)
 
 
+@pytest.mark.parametrize("short,full,M,H,HK", [(672, 672, 673, 48, 16), (70, 64, 5472, 5, 2)])
+def test_gdn_chunked_prep_split_same_bits(q27, dev, short, full, M, H, HK):
+    """The preparing launch with one workgroup per value head (the first `short` tokens) and per key head (all M): the same
+    bits of o in the full chunks that both batches share."""
+    say(f"gdn chunked prep split {short} of {M} tokens H={H} HK={HK}")
+    x, stride, g, beta, planes = cd.gdn_inputs(cd.rng(930 + M), M, H, HK)
+    want, _ = _run(q27, dev, x, stride, g, beta, planes, 0, H, HK, M)
+    got, _ = _run(q27, dev, x[: short * stride].copy(), stride, g[: short * H].copy(), beta[: short * H].copy(), planes, 0,
+                  H, HK, short)
+    n = full * H * 128
+    assert np.array_equal(got[:n].view(np.uint32), want[:n].view(np.uint32))
+
+
 @pytest.mark.parametrize("n", [1, 15, 16, 17, 31])
 def test_gdn_chunked_ragged_rows_inside_a_larger_batch(q27, dev, n):
     """Every row behind the last token is NaN (x, g, beta): a last chunk of n tokens gives the bits of the compact batch,
