@@ -262,7 +262,7 @@ int q27o_qgemv(int type, const uint8_t* raw, int N, int K, const int8_t* xq, con
   for (int n = 0; n < N; n++) {
     const uint8_t* row = raw + (size_t)n * nb * bb;
     for (int c = 0; c < ncols; c++) {
-      /* three columns run as a launch of two columns and one of one */
+      /* three columns are ordered as two columns, then one */
       const int W = q27o_qgemv_waves(type, K, ncols == 3 ? (c < 2 ? 2 : 1) : ncols);
       const int8_t* xr = xq + (size_t)c * K;
       const float* dr = xd + (size_t)c * (K / 32);

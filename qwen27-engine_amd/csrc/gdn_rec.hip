@@ -207,8 +207,8 @@ using namespace q27h;
 
 // Prefill (flip) runs from kChunkMinT tokens on in the chunked form on matrix cores (gdn_chunk.hip), unless the
 // process asked for the sequential, bit-exact kernel. Measured (us, 48 value heads, sequential / chunked): 64 tokens
-// 18.7 / 23.1, 96 tokens 26.4 / 27.0, 128 tokens 33.8 / 30.8, 512 tokens 126 / 77, 2048 tokens 491 / 273, 8192
-// tokens 2008 / 1078.
+// 18.1 / 17.6, 72 20.5 / 21.2, 80 22.4 / 21.2, 96 25.7 / 21.2, 128 33.1 / 24.6, 512 124.8 / 72.4, 2048 490 / 250, 8192 2004 /
+// 1024. The chunked form is faster from 80 tokens on; below 128 callers are promised the checker's bits.
 constexpr int kChunkMinT = 128;
 static std::atomic<int> g_prefill_exact{0};
 

@@ -871,8 +871,8 @@ __device__ __forceinline__ void qgemv_body(Mat m, const int8_t* __restrict__ xq,
     constexpr int G = LutInfo<TYPE>::grid, NM = LutInfo<TYPE>::masks;
     // Every workgroup fills its tables before its first weight, so this is latency on every launch: 16-byte pieces of the
     // codebook and a mask pair in a few operations instead of 4-byte pieces and a loop over the bits (us, T = 1: 1024 x
-    // 5120 IQ2_S 5.3 -> 4.4, IQ1_M 4.8 -> 3.9, IQ3_S 4.4 -> 4.1; 17408 x 5120 IQ2_S 12.7 -> 11.2, IQ2_XS 11.3 -> 10.4, IQ3_S
-    // 12.5 -> 12.2; 32768 x 512 IQ2_S 15.9 -> 9.9). Requesting the weights or activations before the tables measured slower
+    // 5120 IQ2_S 5.2 -> 4.2, IQ1_M 4.8 -> 4.0, IQ3_S 4.3 -> 4.0; 17408 x 5120 IQ2_S 13.0 -> 11.5, IQ2_XS 11.4 -> 10.5, IQ3_S
+    // 11.8 -> 11.5; 32768 x 512 IQ2_S 16.0 -> 10.1). Requesting the weights or activations before the tables measured slower
     // at T = 1 (17408 x 5120 IQ3_S 13.3): a workgroup's weights then wait for the whole fill in registers.
     for (int i = threadIdx.x; i < G / 4; i += blockDim.x) ((u32x4*)lut)[i] = ((const u32x4*)grid_of<TYPE>())[i];
     for (int i = threadIdx.x; i < NM; i += blockDim.x) {
